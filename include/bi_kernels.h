@@ -119,9 +119,9 @@ int bi_matmul_packed(const void* a, int64_t lda, const void* bt, int64_t ldb, co
 
 /* Strided batch of dense matmuls (a [batch][M, K], bt [batch][N, K],
  * out [batch][M, N]; batch strides in elements, 0 broadcasts a or bt): slice i
- * is exactly bi_matmul on the slice's pointers, so its bits equal a 2-D call
- * and do not depend on batch. Same requirements and workspace as bi_matmul
- * (shared by the slices, which run in order on the stream).
+ * has bi_matmul's bits on the slice's pointers, and they do not depend on
+ * batch. Same requirements and workspace as bi_matmul; the slices run in one
+ * grid, or in order on the stream sharing the workspace.
  * Replaces: the reference's fallback for a non-2-D right-hand side
  * (ops.py:46-51, "matmul:non-2d-rhs-or-non-float"); its roadmap's batched
  * matmul (README.md:257-268). */
@@ -129,6 +129,22 @@ int bi_matmul_batched(const void* a, int64_t a_batch_stride, int64_t lda, const 
                       int64_t b_batch_stride, int64_t ldb, void* out, int64_t out_batch_stride,
                       int64_t batch, int64_t M, int64_t N, int64_t K, int dtype, void* ws,
                       size_t ws_bytes, void* stream);
+
+/* The same product with the right-hand side stored row-major: element b[k, n] of
+ * slice i at b[i * b_batch_stride + k * ldb + n] (batch = 1: one matrix), so a
+ * torch.matmul(x, W) with W [K, N], or probabilities times values, needs no
+ * transposed copy. bf16 / fp16; lda, ldb and the batch strides multiples of 8,
+ * 16-byte aligned operands, (K + 512) * ldb < 2^30; when K is not a multiple of
+ * 8 the elements [K, 8 ceil(K / 8)) of every a row must be zero. The bits are
+ * bi_matmul's on the transposed operand. Workspace: fp32 group partials when
+ * one small product splits K (bi_matmul_kn_workspace_bytes).
+ * Replaces: the transposed copy a row-major right-hand side needed before
+ * bi_matmul; the reference reads either layout through strides
+ * (kernels/matmul.py:279-340). */
+size_t bi_matmul_kn_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K);
+int bi_matmul_kn(const void* a, int64_t a_batch_stride, int64_t lda, const void* b, int64_t b_batch_stride,
+                 int64_t ldb, void* out, int64_t out_batch_stride, int64_t batch, int64_t M, int64_t N, int64_t K,
+                 int dtype, void* ws, size_t ws_bytes, void* stream);
 
 /* ---- Affine quantized matmul (MLX packed format) ---------------------------
  * out[M, N] = x[M, K] @ W^T with W[n, k] = T(fmaf(code(n,k), scale, bias)),

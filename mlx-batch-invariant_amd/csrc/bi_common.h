@@ -181,6 +181,21 @@ __device__ __forceinline__ void copy_to_lds16(__amdgpu_buffer_rsrc_t rs, int vof
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t*)lds_block, 16, voffset, 0, 0, 0);
 }
 
+// ds_read_b64_tr_b16: in each 16-lane group, element t % 4 of the 8 bytes read
+// by lane 4 j + t / 4 arrives as slot j of lane t (so lane 4 j + c reading
+// columns 4 c .. 4 c + 3 of row j hands every lane one column of 4 rows).
+// The restrict parameter gives the inlined read an alias scope: without alias
+// information the compiler takes it to overlap every global -> LDS copy in
+// flight and drains them all (s_waitcnt vmcnt(0)) before each read. Ordinary
+// LDS reads carry type information and never get that wait; as for them, the
+// kernel's own stage waits order the reads after the copies they need.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+__device__ __forceinline__ s16x4 lds_read_tr16(lds_s16x4* __restrict p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(p);
+}
+
 // s_waitcnt vmcnt(N) lgkmcnt(0); the empty asm statements keep the compiler
 // from moving memory accesses across it.
 template <int N>

@@ -100,12 +100,56 @@ static_assert(BigTile<4>::kBM == kBigBM && BigTile<4>::kWaves == kBigWaves && Bi
 template <int WM, int BN>
 constexpr int big_threads() { return 64 * BigTile<WM, BN>::kWaves; }
 
-template <typename T, int WM = kBigWavesM, int BN = kBigBN>
+// B operand of the tile kernels (gemm_big, gemm_tall):
+//   kBPlain   bt[n][k], one matrix, K % 64 == 0 (the nn.Linear layout);
+//   kBRows    the same layout, a batch of matrices and any K % 8 == 0;
+//   kBColumns b[k][n] (row-major right-hand side, n contiguous), a batch.
+enum BMode { kBPlain = 0, kBRows = 1, kBColumns = 2 };
+
+// Element strides between the slices of a batch (kBRows, kBColumns).
+struct BatchStride {
+  int64_t a, b, out;
+};
+
+// kBColumns stage: 64 k rows of BN columns, 2 BN bytes each, 16-byte chunk c of
+// row k in slot c ^ kn_key(k). A B fragment (column n of lane r, k 8 q + e) is
+// two ds_read_b64_tr_b16: lane 4 j + c of a quarter reads 4 columns of row
+// 8 q + j (8 q + 4 + j), and the 16 lanes' 4 rows x 32 bytes fall in distinct
+// bank groups under the key (and, for 256-byte rows, so do two quarters').
+template <int BN>
+__device__ __forceinline__ int kn_key(int k) {
+  return 2 * (k & 3) + (BN == 128 ? 8 * ((k >> 3) & 1) : 0);
+}
+template <typename T, int BN>
+__device__ __forceinline__ typename Frag<T>::type kn_frag(const T* stage, int s, int col0, int lane) {
+  const int q = lane / 16, j = lane % 16 / 4, c = lane % 4;
+  const int k0 = 32 * s + 8 * q + j, chunk = col0 / 8 + (c >> 1);
+  const T* p0 = stage + k0 * BN + ((chunk ^ kn_key<BN>(k0)) << 3) + ((c & 1) << 2);
+  const T* p1 = stage + (k0 + 4) * BN + ((chunk ^ kn_key<BN>(k0 + 4)) << 3) + ((c & 1) << 2);
+  const s16x8 v = __builtin_shufflevector(lds_read_tr16((lds_s16x4*)p0), lds_read_tr16((lds_s16x4*)p1), 0, 1, 2, 3, 4,
+                                          5, 6, 7);
+  return __builtin_bit_cast(typename Frag<T>::type, v);
+}
+// Bytes of a kBColumns operand from column n0 of row 0 on: rows at or past K
+// lie beyond it and read as zero. The end is rounded up to a whole 16-byte
+// chunk (chunks are aligned, so the rounding stays in the last element's own
+// 16 bytes).
+__device__ __forceinline__ int kn_bytes(int64_t ldb, int N, int K, int n0) {
+  return (int)(((K - 1) * ldb + (N + 7) / 8 * 8 - n0) * 2);
+}
+
+template <typename T, int WM = kBigWavesM, int BN = kBigBN, int BMODE = kBPlain>
 __global__ __launch_bounds__((big_threads<WM, BN>())) void gemm_big(const T* __restrict__ a, int64_t lda,
                                                                      const T* __restrict__ bt, int64_t ldb,
                                                                      T* __restrict__ out, int M, int N, int K,
-                                                                     int tiles_m, int tiles_n) {
+                                                                     int tiles_m, int tiles_n, BatchStride bs) {
   static_assert(sizeof(T) == 2, "gemm_big: 2-byte element types only");
+  constexpr bool GEN = BMODE != kBPlain, KN = BMODE == kBColumns;
+  if constexpr (GEN) {
+    a += blockIdx.y * bs.a;
+    bt += blockIdx.y * bs.b;
+    out += blockIdx.y * bs.out;
+  }
   typedef typename Frag<T>::type F;
   typedef BigTile<WM, BN> BT;
   constexpr int kBM = BT::kBM, kWavesAll = BT::kWaves, kACop = BT::kACopies, kBCop = BT::kBCopies;
@@ -144,21 +188,39 @@ __global__ __launch_bounds__((big_threads<WM, BN>())) void gemm_big(const T* __r
   const __amdgpu_buffer_rsrc_t ra =
       __builtin_amdgcn_make_buffer_rsrc((void*)(a + (int64_t)m0 * lda), (short)0, (int)(rows_a * lda * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rb =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(bt + (int64_t)n0 * ldb), (short)0, (int)(rows_b * ldb * 2), 0x00020000);
+      KN ? __builtin_amdgcn_make_buffer_rsrc((void*)(bt + n0), (short)0, kn_bytes(ldb, N, K, n0), 0x00020000)
+         : __builtin_amdgcn_make_buffer_rsrc((void*)(bt + (int64_t)n0 * ldb), (short)0, (int)(rows_b * ldb * 2),
+                                             0x00020000);
   const __amdgpu_buffer_rsrc_t r_none = __builtin_amdgcn_make_buffer_rsrc((void*)a, (short)0, 0, 0x00020000);
   const unsigned voa = (unsigned)(((8 * wave + rr) * lda + 8 * ch) * 2);
-  const unsigned vob = (unsigned)(((8 * wave + rr) * ldb + 8 * ch) * 2);
-  // Stage st is 64 k (128 bytes of each row); stages at or past K read as zero.
-  const int kst_valid = K / 64;
+  // kBColumns: copy c of this wave moves the k rows kRowsKn (c kWavesAll + wave) ..
+  constexpr int kCprKn = BN / 8, kRowsKn = 64 / kCprKn;
+  const int kr = kRowsKn * wave + lane / kCprKn;
+  const unsigned vob = KN ? (unsigned)((kr * ldb + 8 * ((lane % kCprKn) ^ kn_key<BN>(kr))) * 2)
+                          : (unsigned)(((8 * wave + rr) * ldb + 8 * ch) * 2);
+  // Stage st is 64 k (128 bytes of each row); stages at or past K read as
+  // zero, and so do the chunks past K of a last partial stage (GEN): their
+  // lanes take an offset outside every resource.
+  const int kst_valid = GEN ? (K + 63) / 64 : K / 64;
+  constexpr unsigned kOutside = 0x80000000u;
   auto copy_a = [&](int st, bool real, int c) {
+    const unsigned off = voa + (unsigned)(c * 8 * kWavesAll * lda * 2);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(real && st < kst_valid ? ra : r_none,
                                              (lds_void_t*)(lds + a_row(st, 8 * (c * kWavesAll + wave))),
-                                             16, voa + (unsigned)(c * 8 * kWavesAll * lda * 2), st * 128, 0, 0);
+                                             16, GEN && 64 * st + 8 * ch >= K ? kOutside : off, st * 128, 0, 0);
   };
   auto copy_b = [&](int st, bool real, int c) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(real && st < kst_valid ? rb : r_none,
-                                             (lds_void_t*)(lds + b_row(st, 8 * (c * kWavesAll + wave))),
-                                             16, vob + (unsigned)(c * 8 * kWavesAll * ldb * 2), st * 128, 0, 0);
+    if constexpr (KN) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(real && st < kst_valid ? rb : r_none,
+                                               (lds_void_t*)(lds + b_row(st, 0) + 512 * (c * kWavesAll + wave)), 16,
+                                               vob + (unsigned)((64 * st + c * kRowsKn * kWavesAll) * ldb * 2),
+                                               0, 0, 0);
+    } else {
+      const unsigned off = vob + (unsigned)(c * 8 * kWavesAll * ldb * 2);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(real && st < kst_valid ? rb : r_none,
+                                               (lds_void_t*)(lds + b_row(st, 8 * (c * kWavesAll + wave))),
+                                               16, GEN && 64 * st + 8 * ch >= K ? kOutside : off, st * 128, 0, 0);
+    }
   };
 
   // Fragment reads: row r of a 16-row block, chunk 4 s + q of step s.
@@ -167,7 +229,8 @@ __global__ __launch_bounds__((big_threads<WM, BN>())) void gemm_big(const T* __r
     f = *reinterpret_cast<const F*>(lds + a_row(st, 16 * TI * wm + 16 * i) + frag_off[s]);
   };
   auto read_b = [&](F& f, int st, int s, int j) {
-    f = *reinterpret_cast<const F*>(lds + b_row(st, 16 * TJ * wn + 16 * j) + frag_off[s]);
+    if constexpr (KN) f = kn_frag<T, BN>(lds + b_row(st, 0), s, 16 * TJ * wn + 16 * j, lane);
+    else f = *reinterpret_cast<const F*>(lds + b_row(st, 16 * TJ * wn + 16 * j) + frag_off[s]);
   };
 
   f32x4 total[TI][TJ], acc[TI][TJ];

@@ -64,11 +64,22 @@ struct TallCfg {
   static __device__ __forceinline__ int slot(int r, int c) { return c ^ (r & (kChunks - 1)); }
 };
 
-template <typename T, int TI, int WM, int WN, int SK, bool SPLIT, int RMAX = 12>
+// BMODE (bi_gemm_big.h) other than kBPlain: a batch of matrices (unsplit:
+// grid.z is the batch; SPLIT: one matrix), any K % 8 == 0, B as bt[n][k] or
+// b[k][n]. 64-k stages and 64 columns, so a stage's B is 64 rows of 128 bytes
+// in either layout.
+template <typename T, int TI, int WM, int WN, int SK, bool SPLIT, int RMAX = 12, int BMODE = kBPlain>
 __global__ __launch_bounds__(256) void gemm_tall(const T* __restrict__ a, int64_t lda, const T* __restrict__ bt,
                                                  int64_t ldb, T* __restrict__ out, float* __restrict__ part,
-                                                 int M, int N, int K, int G, int CG) {
+                                                 int M, int N, int K, int G, int CG, BatchStride bs) {
   static_assert(sizeof(T) == 2, "gemm_tall: 2-byte element types only");
+  constexpr bool GEN = BMODE != kBPlain, KN = BMODE == kBColumns;
+  static_assert(!GEN || (SK == 64 && WN == 4), "gemm_tall: 64 x 64 B stages outside kBPlain");
+  if constexpr (GEN && !SPLIT) {
+    a += blockIdx.z * bs.a;
+    bt += blockIdx.z * bs.b;
+    out += blockIdx.z * bs.out;
+  }
   typedef TallCfg<TI, WM, WN, SK, RMAX> C;
   constexpr int SPG = C::kStagesPerGroup;
   typedef typename Frag<T>::type F;
@@ -83,7 +94,7 @@ __global__ __launch_bounds__(256) void gemm_tall(const T* __restrict__ a, int64_
   const int g_begin = SPLIT ? blockIdx.z * CG : 0;
   const int g_end = SPLIT ? min(G, g_begin + CG) : G;
   const int st0 = SPG * g_begin, nst = SPG * (g_end - g_begin);  // stages of this workgroup
-  const int st_valid = K / SK;                                      // stages inside K (global index)
+  const int st_valid = (K + SK - 1) / SK;                           // stages with k inside K (global index)
 
   // A copy slot c of this wave moves A rows kRowsPerCopy (4 c + wave) .. of
   // the stage, B slot c the same B rows (B rows start at BM in the stage
@@ -98,27 +109,38 @@ __global__ __launch_bounds__(256) void gemm_tall(const T* __restrict__ a, int64_
   const __amdgpu_buffer_rsrc_t ra =
       __builtin_amdgcn_make_buffer_rsrc((void*)(a + (int64_t)m0 * lda), (short)0, (int)(rows_a * lda * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rb =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(bt + (int64_t)n0 * ldb), (short)0, (int)(rows_b * ldb * 2), 0x00020000);
+      KN ? __builtin_amdgcn_make_buffer_rsrc((void*)(bt + n0), (short)0, kn_bytes(ldb, N, K, n0), 0x00020000)
+         : __builtin_amdgcn_make_buffer_rsrc((void*)(bt + (int64_t)n0 * ldb), (short)0, (int)(rows_b * ldb * 2),
+                                             0x00020000);
   const __amdgpu_buffer_rsrc_t r_none = __builtin_amdgcn_make_buffer_rsrc((void*)a, (short)0, 0, 0x00020000);
   const unsigned voa = (unsigned)(((RPC * wave + rr) * lda + 8 * ch) * 2);
-  const unsigned vob = (unsigned)(((RPC * wave + rr) * ldb + 8 * ch) * 2);
+  const int kr = RPC * wave + rr;                                   // kBColumns: k row of copy slot 0
+  const unsigned vob = KN ? (unsigned)((kr * ldb + 8 * ((lane % 8) ^ kn_key<64>(kr))) * 2)
+                          : (unsigned)(((RPC * wave + rr) * ldb + 8 * ch) * 2);
   // Stage st (global index) into buffer st % R. A stage past the workgroup's
   // range or past K goes through the empty resource: no memory traffic, and
   // its buffer is one no stage in flight uses.
   auto copy_stage = [&](int st) {
     const bool real = st - st0 < nst && st < st_valid;
     T* buf = lds + (st % R) * (C::kRowsAlloc * SK);
+    // Chunks past K of a last partial stage (GEN) read as zero: their lanes
+    // take an offset outside every resource.
+    const bool past = GEN && SK * st + 8 * ch >= K;
+    constexpr unsigned kOutside = 0x80000000u;
 #pragma unroll
     for (int c = 0; c < C::kCopiesA; ++c)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(real ? ra : r_none,
                                                (lds_void_t*)(buf + RPC * (4 * c + wave) * SK), 16,
-                                               voa + (unsigned)(4 * RPC * c * lda * 2), st * SK * 2, 0, 0);
+                                               past ? kOutside : voa + (unsigned)(4 * RPC * c * lda * 2),
+                                               st * SK * 2, 0, 0);
 #pragma unroll
     for (int c = 0; c < C::kCopiesB; ++c) {
       const bool live = real && RPC * (4 * c + wave) < C::kBN;
+      const unsigned off = vob + (unsigned)((4 * RPC * c + (KN ? SK * st : 0)) * ldb * 2);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rb : r_none,
                                                (lds_void_t*)(buf + (C::kBM + RPC * (4 * c + wave)) * SK), 16,
-                                               vob + (unsigned)(4 * RPC * c * ldb * 2), st * SK * 2, 0, 0);
+                                               past && !KN ? kOutside : off,
+                                               KN ? 0 : st * SK * 2, 0, 0);
     }
   };
 
@@ -146,7 +168,9 @@ __global__ __launch_bounds__(256) void gemm_tall(const T* __restrict__ a, int64_
     const int p = j % SPG;
 #pragma unroll
     for (int s = 0; s < SK / 32; ++s) {
-      F bf = *reinterpret_cast<const F*>(buf + (C::kBM + 16 * wn) * SK + frag_off(s));
+      F bf;
+      if constexpr (KN) bf = kn_frag<T, 64>(buf + C::kBM * SK, s, 16 * wn, lane);
+      else bf = *reinterpret_cast<const F*>(buf + (C::kBM + 16 * wn) * SK + frag_off(s));
       F af[TI];
 #pragma unroll
       for (int i = 0; i < TI; ++i) af[i] = *reinterpret_cast<const F*>(buf + (16 * TI * wm + 16 * i) * SK + frag_off(s));

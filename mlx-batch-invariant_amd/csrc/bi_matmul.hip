@@ -1,6 +1,6 @@
 // bi_matmul.hip — C ABI of the batch-invariant dense and affine-quantized
 // matmul for gfx950 (kernels and launch policy: bi_matmul_impl.h).
-#include "bi_matmul_impl.h"
+#include "bi_gemm_gen.h"
 
 // ---------------------------------------------------------------------------
 // C ABI
@@ -89,6 +89,15 @@ extern "C" int bi_matmul(const void* a, int64_t lda, const void* bt, int64_t ldb
   hipStream_t st = static_cast<hipStream_t>(stream);
   float* wsf = static_cast<float*>(ws);
   const int Mi = (int)M, Ni = (int)N, Ki = (int)K;
+  // K not a multiple of 64, more than 32 rows: the tall and large tiles with
+  // the chunks past K masked, where the generic LDS tile ran: bf16 [4850, 888]
+  // M = 48 / 200 / 3000 14.7 / 18.3 / 123 -> 13.2 / 12.8 / 58 us, [14300,
+  // 4088] M = 512 266 -> 89 us.
+  if ((dtype == BI_BF16 || dtype == BI_F16) && M > bi::kSplitMMax && K % 64 &&
+      bi::gen_fits(bi::kBRows, lda, ldb, K)) {
+    const auto run = dtype == BI_BF16 ? bi::gen_matmul_bf16 : bi::gen_matmul_f16;
+    return run(bi::kBRows, a, lda, bt, ldb, out, nullptr, 1, bi::BatchStride{0, 0, 0}, Mi, Ni, Ki, st, "bi_matmul");
+  }
   switch (dtype) {
     case BI_BF16: {
       bi::DenseB<bi::bf16> b{static_cast<const bi::bf16*>(bt), ldb, Ni, Ki};
@@ -181,8 +190,9 @@ extern "C" int bi_matmul_packed(const void* a, int64_t lda, const void* bt, int6
 
 // Strided batch of independent matmuls: slice i is exactly bi_matmul on
 // a + i * a_batch_stride, bt + i * b_batch_stride, out + i * out_batch_stride
-// (element strides; 0 broadcasts an operand). The slices run one after the
-// other on the stream and share the workspace.
+// (element strides; 0 broadcasts an operand). Bits never depend on how the
+// slices are launched: one grid over all of them (2-byte types, gen_batch), or
+// one launch after the other on the stream, sharing the workspace.
 extern "C" int bi_matmul_batched(const void* a, int64_t a_batch_stride, int64_t lda, const void* bt,
                                  int64_t b_batch_stride, int64_t ldb, void* out, int64_t out_batch_stride,
                                  int64_t batch, int64_t M, int64_t N, int64_t K, int dtype, void* ws,
@@ -194,6 +204,16 @@ extern "C" int bi_matmul_batched(const void* a, int64_t a_batch_stride, int64_t 
   if (dtype != BI_BF16 && dtype != BI_F16 && dtype != BI_F32)
     return fail(BI_E_UNSUPPORTED, "bi_matmul_batched: unknown dtype %d", dtype);
   const size_t es = dtype == BI_F32 ? 4 : 2;
+  if (es == 2 && M > 0 && M <= 0x7fffffffLL && N > 0 && N <= 0x7fffffffLL && K > 0 && K <= 0x7fffffffLL && K % 8 == 0 &&
+      lda >= K && ldb >= K && a_batch_stride % 8 == 0 && b_batch_stride % 8 == 0 && a && bt && out && aligned16(a) &&
+      aligned16(bt) && bi::gen_fits(bi::kBRows, lda, ldb, K) && bi::gen_batch(batch, M, N, K)) {
+    const int rc = check_common("bi_matmul_batched", M, N, K, out, ws, ws_bytes, true);
+    if (rc) return rc;
+    const auto run = dtype == BI_BF16 ? bi::gen_matmul_bf16 : bi::gen_matmul_f16;
+    return run(bi::kBRows, a, lda, bt, ldb, out, nullptr, batch,
+               bi::BatchStride{a_batch_stride, b_batch_stride, out_batch_stride}, (int)M, (int)N, (int)K,
+               static_cast<hipStream_t>(stream), "bi_matmul_batched");
+  }
   for (int64_t i = 0; i < batch; ++i) {
     const char* ai = static_cast<const char*>(a) + (size_t)(i * a_batch_stride) * es;
     const char* bi_ = static_cast<const char*>(bt) + (size_t)(i * b_batch_stride) * es;
@@ -202,6 +222,49 @@ extern "C" int bi_matmul_batched(const void* a, int64_t a_batch_stride, int64_t 
     if (rc) return rc;
   }
   return BI_OK;
+}
+
+// The right-hand side stored row-major, b[k][n]: the same tiles with the B
+// stages copied as k rows and transposed by the LDS reads.
+extern "C" size_t bi_matmul_kn_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K) {
+  if (batch != 1 || M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
+  const bi::GenPlan p = bi::gen_plan(1, M, N, K, bi::kBColumns);
+  return p.chunks > 1 ? (size_t)((K + bi::kGroupK - 1) / bi::kGroupK * M * N) * sizeof(float) : 0;
+}
+
+extern "C" int bi_matmul_kn(const void* a, int64_t a_batch_stride, int64_t lda, const void* b, int64_t b_batch_stride,
+                            int64_t ldb, void* out, int64_t out_batch_stride, int64_t batch, int64_t M, int64_t N,
+                            int64_t K, int dtype, void* ws, size_t ws_bytes, void* stream) {
+  using namespace bi_host;
+  const char* what = "bi_matmul_kn";
+  if (dtype != BI_BF16 && dtype != BI_F16) return fail(BI_E_UNSUPPORTED, "%s: dtype %d (bf16 and fp16 only)", what, dtype);
+  if (batch < 0 || M < 0 || N <= 0 || K <= 0)
+    return fail(BI_E_INVALID_ARG, "%s: bad shape batch=%lld M=%lld N=%lld K=%lld", what, (long long)batch, (long long)M,
+                (long long)N, (long long)K);
+  if (M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL || M * N > ((int64_t)1 << 46) ||
+      ((M + 63) / 64) * ((N + 63) / 64) > 0x7fffffffLL - 8)
+    return fail(BI_E_UNSUPPORTED, "%s: shape too large", what);
+  if (a_batch_stride < 0 || b_batch_stride < 0 || out_batch_stride < M * N)
+    return fail(BI_E_INVALID_ARG, "%s: negative batch stride or out_batch_stride < M*N", what);
+  if (batch == 0 || M == 0) return BI_OK;
+  if (!a || !b || !out) return fail(BI_E_INVALID_ARG, "%s: null operand", what);
+  if (lda % 8 || ldb % 8 || a_batch_stride % 8 || b_batch_stride % 8 || lda < (K + 7) / 8 * 8 || ldb < N ||
+      !aligned16(a) || !aligned16(b))
+    return fail(BI_E_INVALID_ARG,
+                "%s: needs lda, ldb and batch strides multiples of 8 (lda >= K rounded up to 8, ldb >= N) and 16-byte "
+                "aligned operands (K=%lld lda=%lld ldb=%lld)", what, (long long)K, (long long)lda, (long long)ldb);
+  if (!bi::gen_fits(bi::kBColumns, lda, ldb, K))
+    return fail(BI_E_UNSUPPORTED,
+                "%s: b of K=%lld rows of %lld elements (K + 512 rows must stay below 2^30 elements, lda below 2^22)", what,
+                (long long)K, (long long)ldb);
+  const size_t need = bi_matmul_kn_workspace_bytes(batch, M, N, K);
+  if (need && (!ws || ws_bytes < need || !aligned16(ws)))
+    return fail(BI_E_WORKSPACE, "%s: 16-byte aligned workspace of %zu bytes required, got %zu", what, need,
+                ws ? ws_bytes : (size_t)0);
+  const auto run = dtype == BI_BF16 ? bi::gen_matmul_bf16 : bi::gen_matmul_f16;
+  return run(bi::kBColumns, a, lda, b, ldb, out, ws, batch,
+             bi::BatchStride{a_batch_stride, b_batch_stride, out_batch_stride}, (int)M, (int)N, (int)K,
+             static_cast<hipStream_t>(stream), what);
 }
 
 namespace {

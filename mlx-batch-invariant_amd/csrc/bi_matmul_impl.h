@@ -677,12 +677,13 @@ static void launch_big(const BigPlan& bp, const T* a, int64_t lda, const T* bt, 
   const int work = bp.tiles_m * bp.tiles_n, grid = ((work + 7) / 8) * 8;
   if (bp.form == kBig128x64)
     gemm_big<T, 2, 64><<<grid, big_threads<2, 64>(), 0, st>>>(a, lda, bt, ldb, out, M, N, K, bp.tiles_m,
-                                                              bp.tiles_n);
+                                                              bp.tiles_n, {});
   else if (bp.form == kBig128x128)
     gemm_big<T, 2><<<grid, big_threads<2, kBigBN>(), 0, st>>>(a, lda, bt, ldb, out, M, N, K, bp.tiles_m,
-                                                              bp.tiles_n);
+                                                              bp.tiles_n, {});
   else
-    gemm_big<T><<<grid, big_threads<4, kBigBN>(), 0, st>>>(a, lda, bt, ldb, out, M, N, K, bp.tiles_m, bp.tiles_n);
+    gemm_big<T><<<grid, big_threads<4, kBigBN>(), 0, st>>>(a, lda, bt, ldb, out, M, N, K, bp.tiles_m, bp.tiles_n,
+                                                        {});
 }
 
 // Dense mid-M launch (bi_gemm_tall.h) for 2-byte types: 16 < M <= 1024,
@@ -804,11 +805,13 @@ static void launch_tall2(const T* a, int64_t lda, const DenseB<T>& b, T* out, fl
                          int G, const TallPlan& p, hipStream_t st) {
   dim3 grid(ceil_div(N, 16 * WN), ceil_div(M, 16 * TI * WM), p.chunks);
   if (p.chunks > 1) {
-    gemm_tall<T, TI, WM, WN, SK, true, R><<<grid, 256, 0, st>>>(a, lda, b.bt, b.ldb, out, ws, M, N, K, G, p.cg);
+    gemm_tall<T, TI, WM, WN, SK, true, R><<<grid, 256, 0, st>>>(a, lda, b.bt, b.ldb, out, ws, M, N, K, G, p.cg,
+                                                               {});
     const int64_t MN = (int64_t)M * N;
     fold_groups<T><<<(unsigned)((MN + 255) / 256), 256, 0, st>>>(ws, out, MN, G);
   } else {
-    gemm_tall<T, TI, WM, WN, SK, false, R><<<grid, 256, 0, st>>>(a, lda, b.bt, b.ldb, out, ws, M, N, K, G, G);
+    gemm_tall<T, TI, WM, WN, SK, false, R><<<grid, 256, 0, st>>>(a, lda, b.bt, b.ldb, out, ws, M, N, K, G, G,
+                                                                {});
   }
 }
 

@@ -16,8 +16,9 @@ with more than one group writes fp32 group partials and folds them in a
 second kernel; larger M folds in registers. The choice never changes bits.
 
 B is consumed transposed (``bt[n, k]``, k contiguous), which is how
-``nn.Linear`` stores its weight, so ``x @ W.T`` needs no copy. Other layouts
-and odd K are copied / zero-padded first; neither changes the arithmetic.
+``nn.Linear`` stores its weight, so ``x @ W.T`` needs no copy, or row-major
+(``b[k, n]``, n contiguous, 2-byte types). Other layouts and odd K are copied /
+zero-padded first; neither changes the arithmetic.
 """
 
 from __future__ import annotations
@@ -49,6 +50,37 @@ def _prep_rows(t: torch.Tensor, K8: int) -> torch.Tensor:
     return out
 
 
+_MAX_LD = (1 << 22) - 8          # elements between rows the tile kernels address
+
+
+def _row_major(b: torch.Tensor) -> bool:
+    """A right-hand side [..., K, N] that ``bi_matmul_kn`` reads in place: 2-byte,
+    n-contiguous, 16-byte aligned rows (and slices), small enough for its
+    32-bit offsets."""
+    ld = b.stride(-2)
+    return (b.element_size() == 2 and b.stride(-1) == 1 and ld >= b.shape[-1] and ld % 8 == 0
+            and b.data_ptr() % 16 == 0 and (b.shape[-2] + 512) * ld < 1 << 30 and b.shape[-2] < _MAX_LD
+            and (b.ndim == 2 or (b.stride(0) % 8 == 0 and b.stride(0) >= 0)))
+
+
+def _matmul_kn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> None:
+    """out = a @ b for a [Bt, M, K] and a row-major b [Bt, K, N] (``_row_major``),
+    2-D operands taken as a batch of one."""
+    if a.ndim == 2:
+        a, b, out = a[None], b[None], out[None]
+    Bt, M, K = a.shape
+    N = b.shape[-1]
+    a = _prep_batched(a, (K + 7) // 8 * 8)
+    if a.stride(1) >= _MAX_LD:
+        a = a.contiguous()
+    ws_bytes = _lib.ws_bytes("bi_matmul_kn_workspace_bytes", Bt, M, N, K)
+    ws = _lib.workspace(ws_bytes, a.device)
+    rc = _lib.load().bi_matmul_kn(a.data_ptr(), a.stride(0), a.stride(1), b.data_ptr(), b.stride(0), b.stride(1),
+                                  out.data_ptr(), M * N, Bt, M, N, K, _lib.DTYPE_CODE[a.dtype], _lib.ptr(ws),
+                                  ws_bytes, _lib.stream_of(a))
+    _lib.check(rc, "bi_matmul_kn")
+
+
 def matmul_bt(a2: torch.Tensor, bt: torch.Tensor) -> torch.Tensor:
     """out[M, N] = a2[M, K] @ bt[N, K].T, both already the output dtype, on the GPU."""
     M, K = a2.shape
@@ -59,6 +91,9 @@ def matmul_bt(a2: torch.Tensor, bt: torch.Tensor) -> torch.Tensor:
     if N == 0 or K == 0:
         return out.zero_()
     K8 = (K + 7) // 8 * 8
+    if bt.stride(1) != 1 and _row_major(bt.t()):
+        _matmul_kn(a2, bt.t(), out)
+        return out
     a2 = _prep_rows(a2, K8)
     bt = _prep_rows(bt, K8)
     _lib.load()
@@ -211,7 +246,11 @@ def batch_invariant_bmm(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     if N == 0 or K == 0:
         return out.zero_()
     a3 = a.to(out_dtype).expand(*batch, M, K).reshape(Bt, M, K)
-    bt3 = b.to(out_dtype).expand(*batch, K, N).reshape(Bt, K, N).transpose(1, 2)
+    b3 = b.to(out_dtype).expand(*batch, K, N).reshape(Bt, K, N)
+    if b3.stride(1) != 1 and _row_major(b3):
+        _matmul_kn(a3, b3, out.view(Bt, M, N))
+        return out
+    bt3 = b3.transpose(1, 2)
     K8 = (K + 7) // 8 * 8
     a3 = _prep_batched(a3, K8)
     bt3 = _prep_batched(bt3, K8)

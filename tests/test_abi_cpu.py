@@ -323,3 +323,32 @@ def test_fast_binding_matches_ctypes():
         _lib.qmm_call(*q[:-1])
     with pytest.raises(TypeError):
         _lib.rms_norm_call(*r[:6], "eps", *r[7:])
+
+
+def test_row_major_rhs_checks():
+    """bi_matmul_kn's argument checks, and which operands the Python layer
+    hands it (every other layout keeps the transposed copy)."""
+    import torch
+    from mlx_batch_invariant_amd.kernels.matmul import _row_major
+    lib = _lib.load()
+    p = ctypes.c_void_p(16)
+    call = lambda lda=16, ldb=16, batch=1, M=2, N=16, K=16, dt=2, obs=32, bbs=0: lib.bi_matmul_kn(
+        p, 0, lda, p, bbs, ldb, p, obs, batch, M, N, K, dt, None, 0, None)
+    assert call(dt=0) == -2 and "bf16 and fp16" in _err(lib)
+    assert call(K=0) == -1 and call(N=0) == -1 and call(batch=-1) == -1
+    assert call(M=0) == 0 and call(batch=0) == 0
+    assert call(ldb=12) == -1 and call(ldb=8) == -1 and call(lda=8) == -1 and call(K=17, lda=17) == -1
+    assert call(obs=31) == -1 and call(bbs=4) == -1 and call(bbs=-8) == -1
+    assert call(ldb=1 << 26) == -2 and call(lda=1 << 22) == -2
+    assert lib.bi_matmul_kn_workspace_bytes(1, 1, 1024, 4096) == 16 * 1024 * 4     # 16 chunks of one group
+    assert call(M=1, N=1024, K=4096, lda=4096, ldb=1024, obs=1024) == -3
+    assert lib.bi_matmul_kn_workspace_bytes(2, 1, 1024, 4096) == 0                 # a batch never splits K
+    assert lib.bi_matmul_kn_workspace_bytes(1, 512, 4096, 4096) == 0
+    h = torch.zeros(64, 64, dtype=torch.bfloat16)
+    b3 = torch.zeros(3, 64, 64, dtype=torch.float16)
+    assert _row_major(h) and _row_major(h[:, :40]) and _row_major(h[:, 8:]) and _row_major(b3) and _row_major(b3[:, :7])
+    assert _row_major(b3[:1].expand(5, 64, 64))
+    assert not _row_major(h.t()) and not _row_major(h[:, 4:]) and not _row_major(h.float())
+    assert not _row_major(torch.zeros(64, 60, dtype=torch.bfloat16)) and not _row_major(h[:, ::2])
+    assert not _row_major(h[:1].expand(64, 64)) and not _row_major(torch.zeros(3 * 68, dtype=torch.float16)
+                                                                   .as_strided((3, 8, 8), (68, 8, 1)))

@@ -1,0 +1,107 @@
+"""The dense tiles that take a batch of matrices in one grid, a row-major
+right-hand side and a K that is not a multiple of 64: bit for bit the one-row
+launches on a contiguous transposed copy (which the oracle tests pin), at the
+edges of each tile form, and over the strides the entry points accept."""
+
+import pytest
+import torch
+
+from helpers import DT, bits, gen, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _bi():
+    import mlx_batch_invariant_amd as bi
+    return bi
+
+
+def _one_row(a, bt, r):
+    """Row r of a @ bt.T by the M = 1 launch on padded contiguous operands."""
+    K = a.shape[1]
+    K8 = (K + 7) // 8 * 8
+    ap = torch.zeros((1, K8), dtype=a.dtype, device=a.device)
+    bp = torch.zeros((bt.shape[0], K8), dtype=a.dtype, device=a.device)
+    ap[:, :K], bp[:, :K] = a[r:r + 1], bt
+    return _bi().batch_invariant_matmul(ap, bp.t())
+
+
+def _check_rows(out, a, bt, rows):
+    for r in sorted(set(rows)):
+        assert bits(out[r:r + 1]) == bits(_one_row(a, bt, r)), f"row {r}"
+
+
+# (M, N, K): every tile form's edges, K tails of 8 .. 56 past a stage and short
+# of a group, fewer columns than a tile, split K (few tiles).
+_SHAPES = [(1, 8, 8), (1, 1024, 4096), (31, 64, 72), (33, 96, 264), (64, 200, 1000), (65, 72, 520), (128, 1024, 776),
+           (129, 4096, 1032), (515, 4096, 1064), (300, 14336, 136), (2049, 3080, 1048), (700, 40, 2088)]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", _SHAPES)
+def test_row_major_rhs_equals_transposed(dt, M, N, K):
+    g = gen(M + N + K)
+    a = randn((M, K), DT[dt], g)
+    b = randn((K, N), DT[dt], g, 0.1)
+    got = _bi().batch_invariant_matmul(a, b)
+    _check_rows(got, a, b.t(), [0, M // 2, M - 1, min(M - 1, 63), min(M - 1, 128)])
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [s for s in _SHAPES if s[0] > 32])
+def test_ragged_k_equals_one_row(dt, M, N, K):
+    g = gen(M + 2 * N + K)
+    a = randn((M, K), DT[dt], g)
+    bt = randn((N, K), DT[dt], g, 0.1)
+    got = _bi().batch_invariant_matmul(a, bt.t())
+    _check_rows(got, a, bt, [0, M // 2, M - 1, min(M - 1, 63), min(M - 1, 128)])
+
+
+def test_row_major_views_and_padding():
+    """Offsets, row gaps (which hold NaN), odd K and odd N, non-finite values
+    next to the operands: only the operands' own elements count."""
+    g = gen(5)
+    for M, N, K in [(40, 100, 72), (3, 64, 65), (130, 77, 200), (70, 136, 133)]:
+        a = randn((M, K), torch.bfloat16, g)
+        b = randn((K, N), torch.bfloat16, g)
+        abig = torch.full((M + 2, K + 40), float("nan"), dtype=torch.bfloat16, device="cuda")
+        bbig = torch.full((K + 3, (N + 7) // 8 * 8 + 24), float("nan"), dtype=torch.bfloat16, device="cuda")
+        av, bv = abig[1:M + 1, 8:K + 8], bbig[1:K + 1, 16:N + 16]
+        av.copy_(a)
+        bv.copy_(b)
+        want = _bi().batch_invariant_matmul(a, b.t().contiguous().t())
+        for x in (a, av):
+            for y in (b, bv):
+                assert bits(_bi().batch_invariant_matmul(x, y)) == bits(want), (M, N, K)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("row_major", [False, True])
+@pytest.mark.parametrize("batch,M,N,K", [(2, 1, 64, 8), (5, 17, 96, 264), (3, 64, 72, 520), (48, 33, 64, 136),
+                                         (7, 200, 72, 1032), (70, 128, 128, 64), (130, 300, 40, 72), (9, 520, 520, 200)])
+def test_batched_equals_slices(dt, row_major, batch, M, N, K):
+    g = gen(batch + M + N + K)
+    a = randn((batch, M, K), DT[dt], g)
+    b = randn((batch, K, N) if row_major else (batch, N, K), DT[dt], g, 0.1)
+    got = _bi().batch_invariant_bmm(a, b if row_major else b.transpose(1, 2))
+    for i in sorted({0, 1, batch // 2, batch - 1}):
+        bt = (b[i].t() if row_major else b[i])
+        _check_rows(got[i], a[i], bt, [0, M // 2, M - 1])
+
+
+def test_batched_broadcast_and_sliced_operands():
+    """Zero batch strides, head-sliced views and an odd inner size through
+    torch.matmul's batch rules."""
+    g = gen(11)
+    a = randn((2, 6, 50, 72), torch.float16, g)
+    kv = randn((2, 90, 6, 3, 72), torch.float16, g)          # [B, L, H, parts, D]
+    k, v = kv[:, :, :, 0].permute(0, 2, 3, 1), kv[:, :, :, 1].permute(0, 2, 1, 3)
+    s = _bi().batch_invariant_bmm(a, k)                       # [2, 6, 50, 90]
+    o = _bi().batch_invariant_bmm(s[..., :89], v[..., :89, :])
+    w = randn((72, 40), torch.float16, g)
+    c = _bi().batch_invariant_bmm(a, w)
+    for i, h in [(0, 0), (1, 5)]:
+        assert bits(s[i, h]) == bits(_bi().batch_invariant_matmul(a[i, h], k[i, h]))
+        _check_rows(s[i, h], a[i, h], k[i, h].t(), [0, 49])
+        _check_rows(o[i, h], s[i, h, :, :89], v[i, h, :89].t(), [0, 49])
+        _check_rows(c[i, h], a[i, h], w.t(), [0, 49])
