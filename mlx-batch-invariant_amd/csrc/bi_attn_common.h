@@ -113,16 +113,29 @@ __device__ __forceinline__ int load_uniform_i32(const int32_t* p) {
   return v;
 }
 
+// Four of them with one wait.
+__device__ __forceinline__ void load_uniform4_i32(const int32_t* p0, const int32_t* p1, const int32_t* p2,
+                                                  const int32_t* p3, int (&v)[4]) {
+  asm volatile(
+      "s_load_dword %0, %4, 0x0\n\ts_load_dword %1, %5, 0x0\n\ts_load_dword %2, %6, 0x0\n\t"
+      "s_load_dword %3, %7, 0x0\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(v[0]), "=&s"(v[1]), "=&s"(v[2]), "=&s"(v[3])
+      : "s"(p0), "s"(p1), "s"(p2), "s"(p3)
+      : "memory");
+}
+
 // K/V addressing mode of a kernel instantiation: a contiguous cache, a paged
-// one with pages of 64 keys or more, or one with smaller pages.
-enum KvMode { kKvContig = 0, kKvPaged = 1, kKvRowPaged = 2 };
+// one with pages of 64 keys or more, one with pages of 16 or 32 keys (every
+// aligned 16-key tile lies in one page), or one with smaller pages.
+enum KvMode { kKvContig = 0, kKvPaged = 1, kKvTilePaged = 2, kKvRowPaged = 3 };
 
 // The K/V rows a kernel reads come in aligned 64-key segments (a decode wave's
 // keys of a split, a prefill chunk). Pointer to the first element of segment
 // key `key0` (a multiple of 64) of (sequence b, kv head hk) for kKvContig and
 // kKvPaged (one wave-uniform table read per segment; a page of 64 keys or
 // more holds the whole segment); rows of the segment are then `sl` elements
-// apart. kKvRowPaged kernels resolve every row through kv_row_off instead.
+// apart. kKvTilePaged kernels do the same per 16-key tile (kv_tile),
+// kKvRowPaged ones resolve every row through kv_row_off.
 template <int MODE, typename T, class Args>
 __device__ __forceinline__ const T* kv_segment(const Args& a, const T* base, int64_t sb, int64_t sh, int64_t sl,
                                                int b, int hk, int key0) {
@@ -133,6 +146,19 @@ __device__ __forceinline__ const T* kv_segment(const Args& a, const T* base, int
         clamp_page(load_uniform_i32(a.table + (int64_t)b * a.table_stride + (key0 >> a.page_shift)), a.num_pages);
     return base + (int64_t)page * sb + (int64_t)hk * sh + (int64_t)(key0 & ((1 << a.page_shift) - 1)) * sl;
   }
+}
+
+// Table entry that holds key `pos` of sequence b, and the first element of key
+// pos's row (pos the first key of a 16-key tile) given that entry.
+template <class Args>
+__device__ __forceinline__ const int32_t* kv_entry(const Args& a, int b, int pos) {
+  return a.table + (int64_t)b * a.table_stride + (pos >> a.page_shift);
+}
+template <typename T, class Args>
+__device__ __forceinline__ const T* kv_tile(const Args& a, const T* base, int64_t sb, int64_t sh, int64_t sl, int entry,
+                                            int hk, int pos) {
+  return base + (int64_t)clamp_page(entry, a.num_pages) * sb + (int64_t)hk * sh +
+         (int64_t)(pos & ((1 << a.page_shift) - 1)) * sl;
 }
 
 // Weight of one key of a split: exp2(s - m) if active, exactly 0 otherwise.
@@ -149,36 +175,40 @@ template <> struct PFrag<float> { f32x8 f; };
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
-// PAIRED (bf16): the hi halves of a pair of weights come from one packed
-// conversion; both forms round the same values the same way, so they give the
-// same bits (a kernel picks the one that fits its register budget).
-template <typename T, bool PAIRED = true>
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+
+// Weights 2 j and 2 j + 1 of a step (16-bit types): one packed
+// round-to-nearest-even conversion gives both hi halves; they widen exactly
+// (bf16: the converted bits moved to the top half), so the residuals p - hi
+// are exact differences, rounded once by the second packed conversion.
+template <typename T>
+__device__ __forceinline__ void pfrag_pair(PFrag<T>& r, int j, float p0, float p1) {
+  if constexpr (std::is_same_v<T, bf16>) {
+    const bf16x2_t h = __builtin_convertvector(f32x2_t{p0, p1}, bf16x2_t);
+    const uint32_t hb = __builtin_bit_cast(uint32_t, h);
+    const float h0 = __builtin_bit_cast(float, hb << 16);
+    const float h1 = __builtin_bit_cast(float, hb & 0xffff0000u);
+    const bf16x2_t l = __builtin_convertvector(f32x2_t{p0 - h0, p1 - h1}, bf16x2_t);
+    r.hi[2 * j] = h[0];
+    r.hi[2 * j + 1] = h[1];
+    r.lo[2 * j] = l[0];
+    r.lo[2 * j + 1] = l[1];
+  } else {
+    const f16x2_t h = __builtin_convertvector(f32x2_t{p0, p1}, f16x2_t);
+    const f16x2_t l = __builtin_convertvector(f32x2_t{p0 - (float)h[0], p1 - (float)h[1]}, f16x2_t);
+    r.hi[2 * j] = h[0];
+    r.hi[2 * j + 1] = h[1];
+    r.lo[2 * j] = l[0];
+    r.lo[2 * j + 1] = l[1];
+  }
+}
+
+template <typename T>
 __device__ __forceinline__ PFrag<T> make_pfrag(const float (&p)[8]) {
   PFrag<T> r;
-  if constexpr (PAIRED && std::is_same_v<T, bf16>) {
-    // Per pair of weights: one packed round-to-nearest-even conversion gives
-    // both hi halves; their fp32 values are the converted bits moved to the
-    // top half (an exact widening), so the residuals p - hi are the same
-    // exact differences, rounded once by the second packed conversion.
+  if constexpr (sizeof(T) == 2) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bf16x2_t h = __builtin_convertvector(f32x2_t{p[2 * j], p[2 * j + 1]}, bf16x2_t);
-      const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-      const float h0 = __builtin_bit_cast(float, hb << 16);
-      const float h1 = __builtin_bit_cast(float, hb & 0xffff0000u);
-      const bf16x2_t l = __builtin_convertvector(f32x2_t{p[2 * j] - h0, p[2 * j + 1] - h1}, bf16x2_t);
-      r.hi[2 * j] = h[0];
-      r.hi[2 * j + 1] = h[1];
-      r.lo[2 * j] = l[0];
-      r.lo[2 * j + 1] = l[1];
-    }
-  } else if constexpr (sizeof(T) == 2) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const T h = to_store<T>(p[e]);
-      r.hi[e] = h;
-      r.lo[e] = to_store<T>(p[e] - (float)h);  // exact difference, rounded once
-    }
+    for (int j = 0; j < 4; ++j) pfrag_pair<T>(r, j, p[2 * j], p[2 * j + 1]);
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -210,6 +240,19 @@ __device__ __forceinline__ typename Frag<T>::type ones_frag() {
     f.hi = f.lo;
   }
   return f;
+}
+
+// Maximum over the four lane quarters (lanes l, l ^ 16, l ^ 32, l ^ 48), on
+// the vector ALU: the swaps exchange the odd 16-lane rows (the upper 32 lanes)
+// of one register with the even ones (the lower 32) of the other.
+__device__ __forceinline__ float quarter_max(float m) {
+  const auto larger = [](auto p) {
+    const uint32_t p0 = p[0], p1 = p[1];  // (a bit cast of a vector element would read element 0)
+    return fmaxf(__builtin_bit_cast(float, p0), __builtin_bit_cast(float, p1));
+  };
+  const uint32_t u = __builtin_bit_cast(uint32_t, m);
+  const uint32_t v = __builtin_bit_cast(uint32_t, larger(__builtin_amdgcn_permlane16_swap(u, u, false, false)));
+  return larger(__builtin_amdgcn_permlane32_swap(v, v, false, false));
 }
 
 // ---- split merge -------------------------------------------------------------

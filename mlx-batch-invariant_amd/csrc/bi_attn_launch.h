@@ -82,11 +82,11 @@ __global__ void zero_counter_kernel(U* c) { *c = 0u; }
 // with fewer, the static order costs nothing extra.
 constexpr int kDynMinRounds = 4;
 
-// K/V addressing mode (bi_attn_common.h): contiguous, pages of >= 64 keys, or
-// smaller pages.
+// K/V addressing mode (bi_attn_common.h): contiguous, pages of >= 64 keys, of
+// 16 or 32 keys, or smaller ones.
 template <class Args>
 static int kv_mode(const Args& a) {
-  return !a.table ? kKvContig : a.page_shift >= 6 ? kKvPaged : kKvRowPaged;
+  return !a.table ? kKvContig : a.page_shift >= 6 ? kKvPaged : a.page_shift >= 4 ? kKvTilePaged : kKvRowPaged;
 }
 
 // Paged caches always take the dynamic item order (one instantiation each).
@@ -107,6 +107,7 @@ static int launch_decode_gu(DecodeArgs& a, hipStream_t st) {
   const int64_t most = (int64_t)a.B * a.nsplit * a.Hkv * a.nchunk;
   const int mode = kv_mode(a);
   if (mode == kKvPaged) return launch_decode_paged<T, D, GU, kKvPaged>(a, most, st);
+  if (mode == kKvTilePaged) return launch_decode_paged<T, D, GU, kKvTilePaged>(a, most, st);
   if (mode == kKvRowPaged) return launch_decode_paged<T, D, GU, kKvRowPaged>(a, most, st);
   static int cache[kMaxDev] = {};
   int grid = resident_grid(attn_decode_mfma<T, D, GU, true, kKvContig>, cache);
@@ -147,8 +148,17 @@ int launch_prefill(PrefillArgs& a, hipStream_t st) {
   dim3 grid((unsigned)(8 * ((items + 7) / 8)));
   switch (kv_mode(a)) {
     case kKvPaged: attn_prefill_mfma<T, D, kKvPaged><<<grid, 256, 0, st>>>(a); break;
+    case kKvTilePaged: attn_prefill_mfma<T, D, kKvTilePaged><<<grid, 256, 0, st>>>(a); break;
     case kKvRowPaged: attn_prefill_mfma<T, D, kKvRowPaged><<<grid, 256, 0, st>>>(a); break;
-    default: attn_prefill_mfma<T, D, kKvContig><<<grid, 256, 0, st>>>(a); break;
+    default:
+      if constexpr (sizeof(T) == 2 && D <= 64) {
+        if (items <= kPrefillFewItems) {
+          attn_prefill_mfma<T, D, kKvContig, true><<<grid, 256, 0, st>>>(a);
+          break;
+        }
+      }
+      attn_prefill_mfma<T, D, kKvContig><<<grid, 256, 0, st>>>(a);
+      break;
   }
   return bi_host::launch_status("bi_attn_prefill");
 }

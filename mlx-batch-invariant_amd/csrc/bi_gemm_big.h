@@ -114,11 +114,11 @@ struct BatchStride {
 // kBColumns stage: 64 k rows of BN columns, 2 BN bytes each, 16-byte chunk c of
 // row k in slot c ^ kn_key(k). A B fragment (column n of lane r, k 8 q + e) is
 // two ds_read_b64_tr_b16: lane 4 j + c of a quarter reads 4 columns of row
-// 8 q + j (8 q + 4 + j), and the 16 lanes' 4 rows x 32 bytes fall in distinct
-// bank groups under the key (and, for 256-byte rows, so do two quarters').
+// 8 q + j (8 q + 4 + j), and the 32 lanes of an LDS cycle (8 rows x 32 bytes,
+// k = 0 .. 3 and 8 .. 11 mod 16) fall in distinct banks under the key.
 template <int BN>
 __device__ __forceinline__ int kn_key(int k) {
-  return 2 * (k & 3) + (BN == 128 ? 8 * ((k >> 3) & 1) : 0);
+  return BN == 128 ? 2 * (k & 3) + 8 * ((k >> 3) & 1) : 2 * ((k >> 1) & 1) + 4 * ((k >> 3) & 1);
 }
 template <typename T, int BN>
 __device__ __forceinline__ typename Frag<T>::type kn_frag(const T* stage, int s, int col0, int lane) {

@@ -173,3 +173,44 @@ def test_paged_decode_and_prefill_match_oracle_on_gathered_cache(page_size, toke
         assert_bits_equal(got, want, f"paged Tq={Tq} page={page_size}")
         ref = ora.attention(to_np(q), kg, vg, sc, mask == "causal", "bf16", kv_lens=lq)
         attn_bound_check(got, ref, to_np(q), kg, vg, sc, mask == "causal", "bf16", kv_lens=lq)
+
+
+@pytest.mark.parametrize("dt,D", [("bf16", 32), ("f16", 64), ("bf16", 96), ("f16", 128), ("bf16", 192), ("f16", 256),
+                                  ("f32", 64), ("f32", 192)])
+@pytest.mark.parametrize("page_size", [8, 16, 32, 64])
+def test_paged_tiles_equal_contiguous(dt, D, page_size):
+    """Lengths around the edges of 16-key tiles, 64-key segments and splits, a
+    table that is not whole 64-key segments, spare pages of noise: decode and
+    causal prefill equal the contiguous calls."""
+    bi = _bi()
+    g = gen(D + page_size)
+    lens = torch.tensor([9, 15, 16, 17, 47, 64, 65, 241, 256, 257, 335], dtype=torch.int32)
+    B, Hq, Hkv, L, Tq = len(lens), 4, 2, 335, 9
+    q = randn((B, Hq, Tq, D), DT[dt], g)
+    k = randn((B, Hkv, L, D), DT[dt], g)
+    v = randn((B, Hkv, L, D), DT[dt], g)
+    kp, vp, table = _paginate(k, v, page_size, g, token_major=page_size == 32)
+    lens = lens.cuda()
+    want = bi.batch_invariant_prefill_attention(q, k, v, scale=D ** -0.5, causal=True, kv_lens=lens)
+    assert bits(bi.batch_invariant_paged_attention(q, kp, vp, table, lens, scale=D ** -0.5, mask="causal")) == bits(want)
+    q1 = q[:, :, -1:].contiguous()
+    want = bi.batch_invariant_decode_attention(q1, k, v, scale=D ** -0.5, kv_lens=lens)
+    assert bits(bi.batch_invariant_paged_attention(q1, kp, vp, table, lens, scale=D ** -0.5)) == bits(want)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [32, 64])
+def test_prefill_few_and_many_workgroups_agree(dt, D):
+    """Up to 512 workgroups stage whole splits, more stage 128 keys with three
+    workgroups per CU: the same bits, at lengths around the chunk edges."""
+    bi = _bi()
+    g = gen(D)
+    B, Hq, Hkv, Tq, L = 34, 14, 2, 75, 640
+    q = randn((B, Hq, Tq, D), DT[dt], g)
+    k = randn((B, Hkv, L, D), DT[dt], g)
+    v = randn((B, Hkv, L, D), DT[dt], g)
+    lens = torch.tensor([75, 127, 128, 129, 255, 256, 257, 383, 384, 385, 512, 513, 640] * 3, dtype=torch.int32)[:B].cuda()
+    many = bi.batch_invariant_prefill_attention(q, k, v, scale=D ** -0.5, causal=True, kv_lens=lens)   # 612 workgroups
+    few = torch.cat([bi.batch_invariant_prefill_attention(q[i:i + 17], k[i:i + 17], v[i:i + 17], scale=D ** -0.5,
+                                                          causal=True, kv_lens=lens[i:i + 17]) for i in (0, 17)])
+    assert bits(many) == bits(few)
