@@ -1190,15 +1190,17 @@ static void launch_wg(const T* a, int64_t lda, const BSrc& bsrc, T* out, int M, 
 
 // Mid-M launch (bi_gemm_mid.h) for a quantized B, 2-byte T, K % 256 == 0:
 // 16 < M < kBigMinM at any N, and 4 < M <= 16 with >= 128 blocks of 64
-// columns. Row blocks of 16 MT rows (MT = 1 for M <= 16, 4 for 32 < M <= 64,
-// else 2: M > 64 takes several);
-// when the (column block, row block) tiles are fewer than kMidMinTiles, K is
-// split into chunks of cg groups (per-group fp32 partials in the workspace,
-// then fold_groups) so that about kMidTargetWG workgroups run.
+// columns. Row blocks of 16 MT rows; when the (column block, row block) tiles
+// are too few, K is split into chunks of cg groups (per-group fp32 partials in
+// the workspace, then fold_groups) so that about kMidTargetWG workgroups run.
 constexpr int kMidMinTiles = 160;
 constexpr int kMidTargetWG = 512;
+constexpr int kMidOneRound = 256;   // workgroups of one per CU
+// kMidSplit: M <= 16, and K split into chunks; the others as in mid_plan.
+enum MidForm { kMidSplit = 0, kMidInterleaved, kMidPlain };
 struct MidPlan {
   bool use = false;
+  int form = kMidSplit;
   int mt = 1, mtiles = 1, chunks = 1, cg = 0;
 };
 // 5 <= M <= 16 with at most 2048 columns and 32 or more groups, where the
@@ -1225,23 +1227,81 @@ static inline MidPlan few_columns_plan(int64_t M, int64_t N, int64_t K) {
   return p;
 }
 
+// Whether a call may split K: the shapes for which the workspace query reports
+// the group partials (a fixed part of the C ABI; mid_plan splits fewer).
+static inline bool mid_may_split(int64_t M, int64_t N, int64_t K) {
+  if (M <= 4 || M >= kBigMinM || N <= 0 || K <= 0 || K % kGroupK || K / kGroupK < 2) return false;
+  const int64_t cb = ceil_div(N, 64);
+  if (M <= 16 && cb < 128) return few_columns_plan(M, N, K).use;
+  return cb * ceil_div(M, M <= 16 ? 16 : M <= 32 || M > 64 ? 32 : 64) < kMidMinTiles;
+}
+
+// Rows above 16. The dequantization costs a wave about as much as four row
+// tiles of MFMAs, and what decides a launch's time is whether its workgroups
+// run at once and how often the weight is dequantized again, so (cb = blocks
+// of 64 columns):
+//   * the fewest row tiles per workgroup (1, 2, 4) that keep the grid within
+//     one workgroup per CU run the K-interleaved eight-wave kernel, unless
+//     that leaves fewer than 128 workgroups (more than 32 groups:
+//     mid_may_split), when K is split;
+//   * larger grids run four waves per workgroup, MT = 2 .. 5 row tiles by the
+//     fitted cost 5 + 1.85 MT us per row block (one K = 4096 pass at cb = 224).
+// Both with two A stages and two groups of codes in flight: 16 MT (32 MT) KB
+// of LDS, so two to five workgroups share a CU where a deeper ring held one or
+// two and left a second round. Measured, old plan -> this one, us, 4-bit g64
+// packed / 4-bit g64 MLX layout / 8-bit g128 packed / 8-bit g64 MLX:
+//   [14336, 4096] M = 32   13.7 / 17.7 / 16.8 / 23.1 -> 12.2 / 15.7 / 14.6 / 20.3
+//                 M = 96   28.7 / 42.1 / 45.5 / 62.7 -> 21.1 / 27.7 / 23.4 / 35.7
+//                 M = 160  44.4 / 67.8 / 73.6 / 102  -> 29.7 / 38.9 / 32.4 / 47.2
+//   [4096, 4096]  M = 32   14.3 / 15.8 / 14.9 / 19.3 -> 9.7 / 12.4 / 10.8 / 17.4
+//                 M = 64   16.4 / 17.4 / 16.3 / 19.2 -> 10.3 / 12.9 / 11.3 / 17.9
+//   [4096, 14336] M = 255  57.5 / 79.4 / 79.3 / 117  -> 47.2 / 57.2 / 49.3 / 69.9
+//   [1024, 4096]  M = 255  18.2 / 20.8 / 18.5 / 23.0 -> 9.3 / 12.0 / 10.6 / 17.1
+// K split stays for [1024, 4096] M = 64 (8.4 against 9.3), [4096, 14336] M =
+// 32 (22.5 against 27.4). Interleaving the dequantization with the MFMAs by
+// hand, or the other scheduler and register forms, measured no faster.
 static inline MidPlan mid_plan(int64_t M, int64_t N, int64_t K) {
   MidPlan p;
   if (M <= 4 || M >= kBigMinM || N <= 0 || K <= 0 || K % kGroupK) return p;
   const int G = (int)(K / kGroupK);
-  if (M <= 16 && ceil_div(N, 64) < 128) return few_columns_plan(M, N, K);
-  // 64-row blocks only for 32 < M <= 64; larger M runs several 32-row blocks
-  // (measured faster: more workgroups per CU, each a shallower register file).
+  const int64_t cb = ceil_div(N, 64);
+  if (M <= 16 && cb < 128) return few_columns_plan(M, N, K);
+  p.use = true;
+  p.cg = G;
+  if (M > 16) {
+    int mt = 1;
+    while (mt <= 4 && cb * ceil_div(M, 16 * mt) > kMidOneRound) mt *= 2;
+    const int64_t wg = mt <= 4 ? cb * ceil_div(M, 16 * mt) : 0;
+    const bool whole = G <= 32 ? wg >= 128 : !mid_may_split(M, N, K);
+    if (mt <= 4 && G >= 2 && whole) {
+      p.form = kMidInterleaved;
+      p.mt = mt;
+    } else if (mt > 4 || G < 2) {
+      p.form = kMidPlain;
+      double best = 1e30;
+      for (int t = 2; t <= 5; ++t) {
+        const double cost = ceil_div(M, 16 * t) * (5.0 + 1.85 * t);
+        if (cost < best) {
+          best = cost;
+          p.mt = t;
+        }
+      }
+    }
+    if (p.form != kMidSplit) {
+      p.mtiles = ceil_div(M, 16 * p.mt);
+      return p;
+    }
+  }
+  // M <= 16, or K split: 64-row blocks only for 32 < M <= 64; larger M runs
+  // several 32-row blocks.
   p.mt = M <= 16 ? 1 : (M <= 32 || M > 64) ? 2 : 4;
   p.mtiles = (int)ceil_div(M, 16 * p.mt);
-  const int64_t t = ceil_div(N, 64) * p.mtiles;
-  p.cg = G;
-  if (t < kMidMinTiles && G > 1) {
-    const int want = (int)std::min<int64_t>(G, ceil_div(kMidTargetWG, t));
+  const int64_t t = cb * p.mtiles;
+  if ((t < kMidMinTiles || M > 16) && G > 1) {
+    const int want = (int)std::min<int64_t>(G, std::max<int64_t>(2, ceil_div(kMidTargetWG, t)));
     p.cg = ceil_div(G, want);
     p.chunks = ceil_div(G, p.cg);
   }
-  p.use = true;
   return p;
 }
 
@@ -1254,46 +1314,66 @@ static bool use_mid(const MidPlan& p, int64_t lda, const T* a) {
   }
 }
 
-// Unsplit: an 8-group A ring for 16-row blocks, 4 for 32- and 64-row blocks
-// (a deeper ring for 32 rows measured 7% slower), B loads 8 groups ahead. Split K: short chunks and several workgroups
-// per CU, so a shallow ring and B loads kMidSplitPD groups ahead (a chunk runs
-// in whole rounds of that many groups; the padding groups are not folded).
+// Split K: short chunks and several workgroups per CU, so a shallow ring and B
+// loads kMidSplitPD groups ahead (a chunk runs in whole rounds of that many
+// groups; the padding groups are not folded). M <= 16 unsplit: an 8-group A
+// ring, B loads 8 groups ahead; at most kMidInterleaveMaxTiles workgroups
+// (about one per CU) run the K-interleaved eight-wave kernel (two waves per
+// SIMD), B loads 4 stages ahead; larger grids already put several four-wave
+// workgroups on each CU, where it measured slower.
 constexpr int kMidSplitPD = 2;
-// Unsplit launches of at most this many workgroups (about one per CU) run the
-// K-interleaved eight-wave kernel (two waves per SIMD); larger grids already
-// put several four-wave workgroups on each CU, where it measured slower.
 constexpr int kMidInterleaveMaxTiles = 320;
-// B loads 4 stages ahead, 2 for 64-row blocks (measured at the Llama MLP
-// shape, M = 64: 24.3 against 25.5 us; M = 16 / 32 prefer 4).
-template <int MT> constexpr int mid_interleave_pd() { return MT == 4 ? 2 : 4; }
-template <typename T, class BSrc, int MT, int NA_ONE, int NA_SPLIT>
-static void launch_mid2(const T* a, int64_t lda, const BSrc& bsrc, T* out, float* ws, int M, int N, int K,
-                        int G, const MidPlan& p, hipStream_t st) {
-  constexpr int PD = 8;
+template <typename T, class BSrc, int MT, int NA_SPLIT>
+static void launch_mid_split(const T* a, int64_t lda, const BSrc& bsrc, T* out, float* ws, int M, int N, int K,
+                             int G, const MidPlan& p, hipStream_t st) {
   const dim3 grid(ceil_div(N, 64), p.mtiles, p.chunks);
-  if (p.chunks == 1 && G >= 2 && (int64_t)grid.x * grid.y <= kMidInterleaveMaxTiles) {
-    constexpr int NA2 = MT == 4 ? 2 : 4;
-    gemm_mid2<T, BSrc, MT, mid_interleave_pd<MT>(), NA2, false><<<grid, 512, 0, st>>>(a, lda, bsrc, out, ws, M, N,
-                                                                                      K, G, G);
+  gemm_mid<T, BSrc, MT, kMidSplitPD, NA_SPLIT, true><<<grid, 256, 0, st>>>(a, lda, bsrc, out, ws, M, N, K, G, p.cg);
+  const int64_t MN = (int64_t)M * N;
+  fold_groups<T><<<(unsigned)((MN + 255) / 256), 256, 0, st>>>(ws, out, MN, G);
+}
+
+// M <= 16 (one row tile): a quantized B, or a dense one with few columns and a
+// long K.
+template <typename T, class BSrc>
+static void launch_mid1(const T* a, int64_t lda, const BSrc& bsrc, T* out, float* ws, int M, int N, int K, int G,
+                        const MidPlan& p, hipStream_t st) {
+  if (p.chunks > 1) {
+    launch_mid_split<T, BSrc, 1, 4>(a, lda, bsrc, out, ws, M, N, K, G, p, st);
     return;
   }
-  if (p.chunks > 1) {
-    gemm_mid<T, BSrc, MT, kMidSplitPD, NA_SPLIT, true><<<grid, 256, 0, st>>>(a, lda, bsrc, out, ws, M, N, K, G,
-                                                                             p.cg);
-    const int64_t MN = (int64_t)M * N;
-    fold_groups<T><<<(unsigned)((MN + 255) / 256), 256, 0, st>>>(ws, out, MN, G);
-  } else {
-    gemm_mid<T, BSrc, MT, PD, NA_ONE, false><<<grid, 256, 0, st>>>(a, lda, bsrc, out, ws, M, N, K, G, G);
-  }
+  const dim3 grid(ceil_div(N, 64), p.mtiles);
+  if (G >= 2 && (int64_t)grid.x * grid.y <= kMidInterleaveMaxTiles)
+    gemm_mid2<T, BSrc, 1, 4, 4, false><<<grid, 512, 0, st>>>(a, lda, bsrc, out, ws, M, N, K, G, G);
+  else gemm_mid<T, BSrc, 1, 8, 8, false><<<grid, 256, 0, st>>>(a, lda, bsrc, out, ws, M, N, K, G, G);
 }
 
 template <typename T, class BSrc>
 static void launch_mid(const T* a, int64_t lda, const BSrc& bsrc, T* out, float* ws, int M, int N, int K,
                        int G, const MidPlan& p, hipStream_t st) {
   if constexpr (sizeof(T) == 2 && BSrc::kMeta) {
-    if (p.mt == 1) launch_mid2<T, BSrc, 1, 8, 4>(a, lda, bsrc, out, ws, M, N, K, G, p, st);
-    else if (p.mt == 2) launch_mid2<T, BSrc, 2, 4, 4>(a, lda, bsrc, out, ws, M, N, K, G, p, st);
-    else launch_mid2<T, BSrc, 4, 4, 2>(a, lda, bsrc, out, ws, M, N, K, G, p, st);
+    const dim3 grid(ceil_div(N, 64), p.mtiles);
+    auto inter = [&](auto mt) {
+      gemm_mid2<T, BSrc, decltype(mt)::value, 2, 2, false><<<grid, 512, 0, st>>>(a, lda, bsrc, out, ws, M, N, K, G, G);
+    };
+    auto plain = [&](auto mt) {
+      gemm_mid<T, BSrc, decltype(mt)::value, 2, 2, false><<<grid, 256, 0, st>>>(a, lda, bsrc, out, ws, M, N, K, G, G);
+    };
+    if (p.form == kMidInterleaved) {
+      if (p.mt == 1) inter(std::integral_constant<int, 1>());
+      else if (p.mt == 2) inter(std::integral_constant<int, 2>());
+      else inter(std::integral_constant<int, 4>());
+    } else if (p.form == kMidPlain) {
+      if (p.mt == 2) plain(std::integral_constant<int, 2>());
+      else if (p.mt == 3) plain(std::integral_constant<int, 3>());
+      else if (p.mt == 4) plain(std::integral_constant<int, 4>());
+      else plain(std::integral_constant<int, 5>());
+    } else if (p.mt == 1) {
+      launch_mid1<T, BSrc>(a, lda, bsrc, out, ws, M, N, K, G, p, st);
+    } else if (p.mt == 2) {
+      launch_mid_split<T, BSrc, 2, 4>(a, lda, bsrc, out, ws, M, N, K, G, p, st);
+    } else {
+      launch_mid_split<T, BSrc, 4, 2>(a, lda, bsrc, out, ws, M, N, K, G, p, st);
+    }
   }
 }
 
@@ -1326,7 +1406,7 @@ static int run_gemm(const T* a, int64_t lda, const BSrc& bsrc, T* out, int M, in
       return bi_host::launch_status(what);
     const MidPlan fp = few_columns_plan(M, N, K);
     if (fp.use && lda % 8 == 0 && bi_host::aligned16(a) && bsrc.ldb % 8 == 0 && bi_host::aligned16(bsrc.bt)) {
-      launch_mid2<T, BSrc, 1, 8, 4>(a, lda, bsrc, out, ws, M, N, K, G, fp, st);
+      launch_mid1<T, BSrc>(a, lda, bsrc, out, ws, M, N, K, G, fp, st);
       return bi_host::launch_status(what);
     }
   }
@@ -1482,14 +1562,13 @@ int run_quant_packed_gs(const void* x, int64_t ldx, const uint32_t* w, const voi
     // 4096] M = 32 / 64 15.8-16.1 / 17.8 -> 14.0-14.2 / 16.7 us (same box,
     // bits equal): their per-CU load rate, not the arithmetic, bounds them.
     MidPlan mp = mid_plan(M, N, K);
-    // 33-64 rows that the plan splits over K (64-row blocks, fewer than
-    // kMidMinTiles of them) run unsplit on the copy as 32-row blocks when that
-    // gives at least 128 workgroups: [4096, 4096] / [4096, 8192] / [4096,
-    // 14336] M = 64 17.1 / 22.5 / 37.0 -> 12.5 / 19.8 / 31.0 us, M = 48 14.7
-    // / 20.0 / 33.0 -> 12.8 / 20.5 / 32.2 us (same box, bits equal: the same
-    // group partials, folded in the same order).
+    // 33-64 rows that the plan splits over K (a long K) run unsplit on the
+    // copy as 32-row blocks when that gives at least 128 workgroups: [4096,
+    // 14336] M = 64 32.4 -> 29.9 us (8-bit g128 35.8 -> 31.5; the same group
+    // partials, folded in the same order).
     if (mp.use && mp.mt == 4 && mp.chunks > 1 && (int64_t)ceil_div(N, 64) * ceil_div(M, 32) >= 128 &&
         (int64_t)ceil_div(N, 64) * ceil_div(M, 32) <= kMidInterleaveMaxTiles) {
+      mp.form = kMidInterleaved;
       mp.mt = 2;
       mp.mtiles = ceil_div(M, 32);
       mp.cg = b.G;

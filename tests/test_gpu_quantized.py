@@ -531,3 +531,24 @@ def test_quantized_linear_packed_under_the_mode():
     for p_, c_ in zip(plain, cached):
         assert bits(c_) == bits(p_)
     bi.drop_packed(q.weight)
+
+
+@pytest.mark.parametrize("bits_,gs,packed", [(4, 64, False), (4, 32, True), (8, 128, False), (8, 64, True)])
+@pytest.mark.parametrize("N,K", [(16400, 512), (8200, 768), (4100, 768), (4096, 256), (1000, 2304)])
+def test_quantized_mid_m_row_tiles(bits_, gs, packed, N, K):
+    """17 <= M < 256 at the edges of 1 to 5 row tiles per workgroup: four-wave
+    workgroups (257 column blocks, one K group), the K-interleaved kernel with
+    1, 2 and 4 row tiles (129 and 65 blocks, an odd group count), split K (16
+    blocks). First, middle and last rows equal the same rows computed alone."""
+    bi = _bi()
+    wq, s, b = (t.cuda() for t in _qweights(N, K, bits_, gs, "bf16", seed=bits_ + gs + N))
+    x = randn((255, K), torch.bfloat16, gen(N + K))
+    run = lambda xx: bi.batch_invariant_quantized_matmul(xx, wq, s, b, group_size=gs, bits=bits_)
+    alone = {r: bits(run(x[r:r + 1])) for r in {0, 16, 32, 47, 64, 79, 80, 96, 128, 159, 254}}
+    if packed:
+        bi.cache_packed(wq, s, b, group_size=gs, bits=bits_)
+    for M in (17, 33, 48, 65, 80, 81, 97, 129, 160, 255):
+        got = run(x[:M])
+        for r in [q for q in alone if q < M]:
+            assert bits(got[r:r + 1]) == alone[r], (M, r)
+    bi.drop_packed(wq)
