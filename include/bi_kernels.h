@@ -331,6 +331,22 @@ int bi_attn_prefill_per_key(const void* q, const void* k, const void* v, const i
                             int64_t D, const int64_t* strides, int causal, float scale, int64_t split_size,
                             int dtype, void* stream);
 
+/* Rotary embedding of a block's queries and keys and the write of its keys and
+ * values into the K/V cache, in one launch. q [B, T, Hq, D], k / v [B, T, Hkv,
+ * D] with heads contiguous and q_row / k_row / v_row elements between tokens;
+ * cos / sin contiguous [T, D / 2] of the tokens' positions; with the halves x1,
+ * x2 of a head y1 = T(T(x1 cos) - T(x2 sin)), y2 = T(T(x2 cos) + T(x1 sin)).
+ * q_out contiguous [B, Hq, T, D]; keys and values of token t go to row pos + t
+ * (pos + T <= max_len) of the caches, whose (batch, head, position) element
+ * strides are strides[0..2] (k) and strides[3..5] (v), d contiguous. D % 16 ==
+ * 0, 16-byte aligned rows; outputs must not overlap inputs.
+ * Replaces: nothing in the reference's kernels (its models rotate through
+ * mx.fast.rope, harness/model_sweep.py:62-108). */
+int bi_rope_cache(const void* q, int64_t q_row, const void* k, int64_t k_row, const void* v, int64_t v_row,
+                  const void* cos, const void* sin, void* q_out, void* k_cache, void* v_cache, int64_t B, int64_t T,
+                  int64_t Hq, int64_t Hkv, int64_t D, int64_t pos, int64_t max_len, const int64_t* strides, int dtype,
+                  void* stream);
+
 /* Diagnostic, no counterpart in the reference: y[i] = the hardware base-2
  * exponential (v_exp_f32) of x[i], n >= 0 floats, device pointers, on the
  * stream. It is the instruction the matrix-core attention kernels compute

@@ -74,6 +74,9 @@ _SIGNATURES = {
     "bi_attn_prefill_paged": (ctypes.c_int, [_vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64,
                                              _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_i64), ctypes.c_int,
                                              ctypes.c_float, ctypes.c_int, _vp]),
+    "bi_rope_cache": (ctypes.c_int, [_vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64,
+                                     _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_i64), ctypes.c_int,
+                                     _vp]),
     "bi_exp2_f32": (ctypes.c_int, [_vp, _vp, _c_i64, _vp]),
     "bi_stream_read": (ctypes.c_int, [_vp, _c_i64, _vp, ctypes.c_uint32, _vp]),
     "bi_quantized_dequantize": (ctypes.c_int, [_vp, _vp, _vp, _vp, _c_i64, _c_i64, ctypes.c_int, ctypes.c_int,

@@ -24,6 +24,7 @@ import torch
 import torch.nn.functional as F
 from torch.nn.attention.bias import causal_lower_right
 
+from . import _lib, _mode
 from .nn import QuantizedLinear
 
 
@@ -74,14 +75,16 @@ class Block(torch.nn.Module):
         cfg = self.cfg
         B, T, _ = x.shape
         hn = self.attn_norm(x)
-        q = self.q(hn).view(B, T, cfg.heads, cfg.head_dim).transpose(1, 2)
-        k = self.k(hn).view(B, T, cfg.kv_heads, cfg.head_dim).transpose(1, 2)
-        v = self.v(hn).view(B, T, cfg.kv_heads, cfg.head_dim).transpose(1, 2)
-        q = _rope(q, cos, sin)
-        k = _rope(k, cos, sin)
+        q = self.q(hn).view(B, T, cfg.heads, cfg.head_dim)
+        k = self.k(hn).view(B, T, cfg.kv_heads, cfg.head_dim)
+        v = self.v(hn).view(B, T, cfg.kv_heads, cfg.head_dim)
         kc, vc = cache
-        kc[:, :, pos:pos + T] = k
-        vc[:, :, pos:pos + T] = v
+        if _fused_rope_ok(q, k, v, cos, sin, kc, vc, pos):
+            q = rope_cache(q, k, v, cos, sin, kc, vc, pos)
+        else:
+            q = _rope(q.transpose(1, 2), cos, sin)
+            kc[:, :, pos:pos + T] = _rope(k.transpose(1, 2), cos, sin)
+            vc[:, :, pos:pos + T] = v.transpose(1, 2)
         L = pos + T
         if T == 1:
             mask = {}
@@ -99,6 +102,40 @@ class Block(torch.nn.Module):
 def _rope(x, cos, sin):
     x1, x2 = x[..., : x.shape[-1] // 2], x[..., x.shape[-1] // 2:]
     return torch.cat([x1 * cos - x2 * sin, x2 * cos + x1 * sin], dim=-1)
+
+
+def _fused_rope_ok(q, k, v, cos, sin, kc, vc, pos) -> bool:
+    """Whether ``rope_cache`` takes a block's tensors (under the mode, on the
+    GPU, one dtype, 16-byte aligned rows, no gradient to record)."""
+    ts = (q, k, v, cos, sin, kc, vc)
+    dt, D = q.dtype, q.shape[-1]
+    unit = 16 // q.element_size() if dt in _lib.FLOAT_DTYPES else 0
+    if not unit or not _mode.is_batch_invariant_mode_enabled() or D % 16 or pos + q.shape[1] > min(kc.shape[2], vc.shape[2]):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    if any(type(t) is not torch.Tensor or not t.is_cuda or t.dtype != dt or t.device != q.device or t.data_ptr() % 16
+           for t in ts):
+        return False
+    # rows [b, t] at one stride with contiguous heads; contiguous tables; caches with contiguous d
+    rows = all(t.is_contiguous() for t in (q, k, v, cos, sin))
+    return rows and all(c.stride(3) == 1 and all(s % unit == 0 for s in c.stride()[:3])
+                        and c.shape[0] == q.shape[0] and c.shape[1] == k.shape[2] and c.shape[3] == D for c in (kc, vc))
+
+
+def rope_cache(q, k, v, cos, sin, kc, vc, pos):
+    """One launch (``bi_rope_cache``) for ``_rope`` of q and k and the writes of
+    the rotated keys and the values into rows ``pos ..`` of the caches: the bits
+    of those elementwise ops. Returns q rotated, ``[B, heads, T, D]``."""
+    B, T, Hq, D = q.shape
+    Hkv = k.shape[2]
+    out = torch.empty((B, Hq, T, D), dtype=q.dtype, device=q.device)
+    strides = (_lib._c_i64 * 6)(*kc.stride()[:3], *vc.stride()[:3])
+    rc = _lib.load().bi_rope_cache(q.data_ptr(), Hq * D, k.data_ptr(), Hkv * D, v.data_ptr(), Hkv * D, cos.data_ptr(),
+                                   sin.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), B, T, Hq, Hkv, D, pos,
+                                   min(kc.shape[2], vc.shape[2]), strides, _lib.DTYPE_CODE[q.dtype], _lib.stream_of(q))
+    _lib.check(rc, "bi_rope_cache")
+    return out
 
 
 class LlamaShaped(torch.nn.Module):

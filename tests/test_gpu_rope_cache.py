@@ -1,0 +1,48 @@
+"""RoPE and the K/V cache writes in one launch against the elementwise ops, bit
+for bit, over types, head sizes, token counts and cache layouts."""
+
+import pytest
+import torch
+
+from helpers import DT, bits, gen, randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("B,T,Hq,Hkv,D,pos", [(1, 1, 32, 8, 128, 0), (3, 5, 4, 2, 64, 11), (2, 37, 3, 1, 16, 3),
+                                              (5, 1, 14, 2, 96, 62)])
+@pytest.mark.parametrize("token_major", [False, True])
+def test_rope_cache_equals_elementwise(dt, B, T, Hq, Hkv, D, pos, token_major):
+    from mlx_batch_invariant_amd import set_batch_invariant_mode
+    from mlx_batch_invariant_amd.llama import _fused_rope_ok, _rope, rope_cache
+    g = gen(B + T + D)
+    q, k, v = (randn((B, T, h, D), DT[dt], g, 3.0) for h in (Hq, Hkv, Hkv))
+    ang = torch.rand((T, D // 2), generator=g) * 6.3
+    cos, sin = ang.cos().to(DT[dt]).cuda(), ang.sin().to(DT[dt]).cuda()
+    L = pos + T + 2
+    shape = (B + 1, L, Hkv, D) if token_major else (B + 1, Hkv, L, D)
+    base = [randn(shape, DT[dt], g) for _ in range(2)]
+    view = lambda c: (c.permute(0, 2, 1, 3) if token_major else c)[1:]       # a slice of a larger cache
+    want = [c.clone() for c in base]
+    qw = _rope(q.transpose(1, 2), cos, sin)
+    view(want[0])[:, :, pos:pos + T] = _rope(k.transpose(1, 2), cos, sin)
+    view(want[1])[:, :, pos:pos + T] = v.transpose(1, 2)
+    assert not _fused_rope_ok(q, k, v, cos, sin, view(base[0]), view(base[1]), pos)      # outside the mode
+    with set_batch_invariant_mode():
+        assert _fused_rope_ok(q, k, v, cos, sin, view(base[0]), view(base[1]), pos)
+        assert not _fused_rope_ok(q, k, v, cos, sin, view(base[0]), view(base[1]), L)    # past the cache
+        assert not _fused_rope_ok(q.transpose(1, 2).contiguous().transpose(1, 2), k, v, cos, sin, view(base[0]),
+                                  view(base[1]), pos) or T == 1
+    got = rope_cache(q, k, v, cos, sin, view(base[0]), view(base[1]), pos)
+    assert bits(got) == bits(qw)
+    for a, b in zip(base, want):
+        assert bits(a) == bits(b)                                            # every other row untouched
+
+
+def test_rope_cache_rejects():
+    from mlx_batch_invariant_amd.llama import rope_cache
+    q, k = torch.zeros(1, 2, 4, 64, device="cuda"), torch.zeros(1, 2, 2, 64, device="cuda")
+    cs, c = torch.zeros(2, 32, device="cuda"), torch.zeros(1, 2, 3, 64, device="cuda")
+    with pytest.raises(ValueError, match="bad shape"):
+        rope_cache(q, k, k, cs, cs, c, c.clone(), 2)                         # rows past the cache
