@@ -146,6 +146,16 @@ int bi_matmul_kn(const void* a, int64_t a_batch_stride, int64_t lda, const void*
                  int64_t ldb, void* out, int64_t out_batch_stride, int64_t batch, int64_t M, int64_t N, int64_t K,
                  int dtype, void* ws, size_t ws_bytes, void* stream);
 
+/* Rows copied into contiguous rows of cols_out elements, zero past cols: row r of
+ * slice b from in + (b * batch_stride + r * row_stride) elements, inner stride
+ * 1, any alignment, to out[b][r] (16-byte aligned, cols_out * elem_bytes a
+ * multiple of 16). elem_bytes 2 or 4. What the matmul entry points take in
+ * place of an operand whose rows they cannot read.
+ * Replaces: nothing in the reference (its kernels mask odd sizes,
+ * kernels/matmul.py:81-190). */
+int bi_pad_rows(const void* in, int64_t batch_stride, int64_t row_stride, void* out, int64_t batch, int64_t rows,
+                int64_t cols, int64_t cols_out, int elem_bytes, void* stream);
+
 /* ---- Affine quantized matmul (MLX packed format) ---------------------------
  * out[M, N] = x[M, K] @ W^T with W[n, k] = T(fmaf(code(n,k), scale, bias)),
  * code(n, k) = (w[n, k*bits/32] >> (bits * (k % (32/bits)))) & (2^bits - 1),

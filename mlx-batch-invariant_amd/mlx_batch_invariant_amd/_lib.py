@@ -49,6 +49,7 @@ _SIGNATURES = {
     "bi_matmul_kn_workspace_bytes": (ctypes.c_size_t, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "bi_matmul_kn": (ctypes.c_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _c_i64,
                                     _c_i64, _c_i64, ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
+    "bi_pad_rows": (ctypes.c_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int, _vp]),
     "bi_quantized_matmul_workspace_bytes": (ctypes.c_size_t, [_c_i64, _c_i64, _c_i64]),
     "bi_quantized_matmul": (ctypes.c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64,
                                            ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, ctypes.c_size_t, _vp]),

@@ -40,11 +40,24 @@ def _kcontig(t: torch.Tensor) -> bool:
             and t.stride(0) >= t.shape[-1])
 
 
+def _pad_rows(t: torch.Tensor, C: int) -> torch.Tensor:
+    """A contiguous copy of t [..., R, c] (2 or 3 dims, unit last stride, any
+    alignment) with rows zero-padded to C elements, in one pass."""
+    out = torch.empty((*t.shape[:-1], C), dtype=t.dtype, device=t.device)
+    batch, bs = (t.shape[0], t.stride(0)) if t.ndim == 3 else (1, 0)
+    rc = _lib.load().bi_pad_rows(t.data_ptr(), bs, t.stride(-2), out.data_ptr(), batch, t.shape[-2], t.shape[-1], C,
+                                 t.element_size(), _lib.stream_of(t))
+    _lib.check(rc, "bi_pad_rows")
+    return out
+
+
 def _prep_rows(t: torch.Tensor, K8: int) -> torch.Tensor:
     """[R, K] -> [R, K8] k-contiguous, 16-byte aligned rows, zero-padded to K8."""
     K = t.shape[1]
     if K8 == K and _kcontig(t):
         return t
+    if t.stride(1) == 1:
+        return _pad_rows(t, K8)
     out = torch.zeros((t.shape[0], K8), dtype=t.dtype, device=t.device)
     out[:, :K] = t
     return out
@@ -63,13 +76,27 @@ def _row_major(b: torch.Tensor) -> bool:
             and (b.ndim == 2 or (b.stride(0) % 8 == 0 and b.stride(0) >= 0)))
 
 
+def _as_row_major(b: torch.Tensor) -> torch.Tensor | None:
+    """A right-hand side [..., K, N] for ``_matmul_kn``: b itself, a copy with
+    aligned rows when only its row length or alignment is in the way, else
+    None (the transposed copy)."""
+    if b.stride(-1) != 1 or b.element_size() != 2 or b.shape[-1] == 1:
+        return None
+    if _row_major(b):
+        return b
+    N8 = (b.shape[-1] + 7) // 8 * 8
+    if (b.shape[-2] + 512) * N8 >= 1 << 30 or b.shape[-2] >= _MAX_LD:
+        return None
+    return _pad_rows(b, N8)
+
+
 def _matmul_kn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> None:
-    """out = a @ b for a [Bt, M, K] and a row-major b [Bt, K, N] (``_row_major``),
-    2-D operands taken as a batch of one."""
+    """out = a @ b for a [Bt, M, K] and a row-major b [Bt, K, N] (``_row_major``;
+    its rows may be padded past out's N), 2-D operands taken as a batch of one."""
     if a.ndim == 2:
         a, b, out = a[None], b[None], out[None]
     Bt, M, K = a.shape
-    N = b.shape[-1]
+    N = out.shape[-1]
     a = _prep_batched(a, (K + 7) // 8 * 8)
     if a.stride(1) >= _MAX_LD:
         a = a.contiguous()
@@ -91,9 +118,11 @@ def matmul_bt(a2: torch.Tensor, bt: torch.Tensor) -> torch.Tensor:
     if N == 0 or K == 0:
         return out.zero_()
     K8 = (K + 7) // 8 * 8
-    if bt.stride(1) != 1 and _row_major(bt.t()):
-        _matmul_kn(a2, bt.t(), out)
-        return out
+    if bt.stride(1) != 1:
+        b = _as_row_major(bt.t())
+        if b is not None:
+            _matmul_kn(a2, b, out)
+            return out
     a2 = _prep_rows(a2, K8)
     bt = _prep_rows(bt, K8)
     _lib.load()
@@ -212,6 +241,8 @@ def _prep_batched(t: torch.Tensor, K8: int) -> torch.Tensor:
           and (t.stride(0) * es) % 16 == 0 and t.data_ptr() % 16 == 0)
     if ok:
         return t
+    if t.stride(2) == 1:
+        return _pad_rows(t, K8)
     out = torch.zeros((Bt, R, K8), dtype=t.dtype, device=t.device)
     out[:, :, :K] = t
     return out
@@ -247,9 +278,11 @@ def batch_invariant_bmm(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
         return out.zero_()
     a3 = a.to(out_dtype).expand(*batch, M, K).reshape(Bt, M, K)
     b3 = b.to(out_dtype).expand(*batch, K, N).reshape(Bt, K, N)
-    if b3.stride(1) != 1 and _row_major(b3):
-        _matmul_kn(a3, b3, out.view(Bt, M, N))
-        return out
+    if b3.stride(1) != 1:
+        bn = _as_row_major(b3)
+        if bn is not None:
+            _matmul_kn(a3, bn, out.view(Bt, M, N))
+            return out
     bt3 = b3.transpose(1, 2)
     K8 = (K + 7) // 8 * 8
     a3 = _prep_batched(a3, K8)

@@ -105,3 +105,34 @@ def test_batched_broadcast_and_sliced_operands():
         _check_rows(s[i, h], a[i, h], k[i, h].t(), [0, 49])
         _check_rows(o[i, h], s[i, h, :, :89], v[i, h, :89].t(), [0, 49])
         _check_rows(c[i, h], a[i, h], w.t(), [0, 49])
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("shape,cut", [((1, 1), (0, 0)), ((3, 7), (0, 0)), ((5, 9), (1, 3)), ((130, 65), (2, 1)),
+                                       ((2, 33, 100), (1, 5)), ((70, 3, 31), (0, 2))])
+def test_pad_rows_copies_exactly(dt, shape, cut):
+    """Every row length and alignment, views with gaps and offsets (the gaps
+    hold NaN), a broadcast batch: the rows, then zeros."""
+    from mlx_batch_invariant_amd.kernels.matmul import _pad_rows
+    big = torch.full((*shape[:-1], shape[-1] + 11), float("nan"), dtype=DT[dt], device="cuda")
+    t = big[..., cut[1]:cut[1] + shape[-1]][..., cut[0]:, :]
+    t.copy_(randn(tuple(t.shape), DT[dt], gen(shape[-1])))
+    for C in ((shape[-1] + 7) // 8 * 8, (shape[-1] + 7) // 8 * 8 + 16):
+        want = torch.zeros((*t.shape[:-1], C), dtype=DT[dt], device="cuda")
+        want[..., :shape[-1]] = t
+        assert bits(_pad_rows(t, C)) == bits(want)
+    if t.ndim == 2:
+        assert bits(_pad_rows(t.expand(4, *t.shape), C)) == bits(want.expand(4, *want.shape))
+
+
+def test_odd_columns_row_major():
+    """b [K, N] with an odd N or an unaligned base takes a row-padded copy."""
+    g = gen(2)
+    for M, N, K in [(1, 33, 100), (70, 1001, 264), (300, 65, 72)]:
+        a, b = randn((M, K), torch.float16, g), randn((K, N + 3), torch.float16, g)
+        for y in (b[:, :N], b[:, 3:]):
+            got = _bi().batch_invariant_matmul(a, y)
+            _check_rows(got, a, y.t(), [0, M - 1])
+        a3, b3 = randn((3, M, K), torch.float16, g), randn((3, K, N), torch.float16, g)
+        got = _bi().batch_invariant_bmm(a3, b3)
+        _check_rows(got[2], a3[2], b3[2].t(), [0, M - 1])
