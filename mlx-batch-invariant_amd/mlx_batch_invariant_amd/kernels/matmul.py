@@ -201,6 +201,35 @@ def drop_packed_weight(weight: torch.Tensor) -> None:
         del _PACKED[weight.data_ptr()]
 
 
+def _matmul_direct(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor | None:
+    """``bi_matmul`` for the common call: 2-D GPU operands of one dtype, ``b`` a
+    transposed view of k-contiguous rows (``W.T``), both readable in place, no
+    repacked copy to look up; None for any other call. The checks of the general
+    path on values read once, without the transposed view it builds: a call
+    whose kernel takes 4.5 us (bf16 [1, 896] @ [4864, 896].T) 11.1 -> 7.7 us."""
+    if a.ndim != 2 or b.ndim != 2 or not a.is_cuda or not b.is_cuda:
+        return None
+    dt = a.dtype
+    code = _lib.DTYPE_CODE.get(dt)
+    M, K = a.shape
+    Kb, N = b.shape
+    if code is None or b.dtype != dt or K != Kb or M == 0 or N == 0 or K == 0 or K % 8 or (_PACKED and M <= PACKED_MAX_M):
+        return None
+    lda, a1 = a.stride()
+    b0, ldb = b.stride()
+    pa, pb = a.data_ptr(), b.data_ptr()
+    if a1 != 1 or b0 != 1 or lda < K or ldb < K or lda % 8 or ldb % 8 or (pa | pb) % 16:
+        return None
+    _lib.load()
+    out = torch.empty((M, N), dtype=dt, device=a.device)
+    ws_bytes = _lib.ws_bytes("bi_matmul_workspace_bytes", M, N, K)
+    ws = _lib.workspace(ws_bytes, a.device) if ws_bytes else None
+    rc = _lib.matmul_call(pa, lda, pb, ldb, out.data_ptr(), M, N, K, code, _lib.ptr(ws), ws_bytes, _lib.stream_of(a))
+    if rc:
+        _lib.check(rc, "bi_matmul")
+    return out
+
+
 def batch_invariant_matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """``a @ b`` for 2-D ``b`` with a batch-invariant reduction order.
 
@@ -209,6 +238,9 @@ def batch_invariant_matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     fp32; the output dtype is the promoted input dtype
     (reference: kernels/matmul.py:317-340).
     """
+    out = _matmul_direct(a, b)
+    if out is not None:
+        return out
     if b.ndim != 2:
         raise ValueError("batch_invariant_matmul: b must be 2-D")
     if a.ndim < 1:

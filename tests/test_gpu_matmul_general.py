@@ -136,3 +136,30 @@ def test_odd_columns_row_major():
         a3, b3 = randn((3, M, K), torch.float16, g), randn((3, K, N), torch.float16, g)
         got = _bi().batch_invariant_bmm(a3, b3)
         _check_rows(got[2], a3[2], b3[2].t(), [0, M - 1])
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 8), (1, 33, 264), (17, 64, 256), (33, 130, 520), (300, 65, 72)])
+def test_direct_call_equals_general(dt, M, N, K):
+    """x @ W.T passed on at once, and the same product through the general path:
+    whole operands, aligned row slices with gaps, and what is not taken at once
+    (an odd base, row strides of 4 mod 8, a row stride below K, mixed types)."""
+    from mlx_batch_invariant_amd.kernels.matmul import _matmul_direct, matmul_bt
+    g = gen(4)
+    a0, w0 = randn((M, K), DT[dt], g), randn((N, K), DT[dt], g)
+    x, w = randn((M + 1, K + 20), DT[dt], g), randn((N + 1, K + 20), DT[dt], g)
+    want = matmul_bt(a0, w0)
+    assert bits(_matmul_direct(a0, w0.t())) == bits(want)
+    x8, w8 = randn((M + 1, K + 24), DT[dt], g), randn((N + 1, K + 24), DT[dt], g)
+    a, wv = x8[1:, 8:8 + K], w8[1:, 16:16 + K]
+    a.copy_(a0)
+    wv.copy_(w0)
+    assert bits(_matmul_direct(a, wv.t())) == bits(want)
+    assert bits(_bi().batch_invariant_matmul(a, wv.t())) == bits(want)
+    if dt != "f32":
+        for y, v in [(x[1:, 1:1 + K], w0), (a0, w[1:, 4:4 + K])]:
+            assert _matmul_direct(y, v.t()) is None
+            assert bits(_bi().batch_invariant_matmul(y, v.t())) == bits(matmul_bt(y.contiguous(), v.contiguous()))
+    assert _matmul_direct(a0[:1].expand(2, K), w0.t()) is None
+    assert _matmul_direct(a0, w0.t().double()) is None and _matmul_direct(a0.cpu(), w0.cpu().t()) is None
+    assert bits(_bi().batch_invariant_matmul(a0[:1].expand(2, K), w0.t())[1]) == bits(matmul_bt(a0[:1], w0)[0])
