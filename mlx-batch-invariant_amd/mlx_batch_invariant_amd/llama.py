@@ -106,9 +106,13 @@ def _rope(x, cos, sin):
 
 def _fused_rope_ok(q, k, v, cos, sin, kc, vc, pos) -> bool:
     """Whether ``rope_cache`` takes a block's tensors (under the mode, on the
-    GPU, one dtype, 16-byte aligned rows, no gradient to record)."""
+    GPU, one dtype, 16-byte aligned rows, one table row per token, no gradient
+    to record). Tables that broadcast (one position per sequence, one row for
+    every token) take the elementwise ops."""
     ts = (q, k, v, cos, sin, kc, vc)
     dt, D = q.dtype, q.shape[-1]
+    if not _tables_fit(q, cos, sin):
+        return False
     unit = 16 // q.element_size() if dt in _lib.FLOAT_DTYPES else 0
     if not unit or not _mode.is_batch_invariant_mode_enabled() or D % 16 or pos + q.shape[1] > min(kc.shape[2], vc.shape[2]):
         return False
@@ -123,12 +127,20 @@ def _fused_rope_ok(q, k, v, cos, sin, kc, vc, pos) -> bool:
                         and c.shape[0] == q.shape[0] and c.shape[1] == k.shape[2] and c.shape[3] == D for c in (kc, vc))
 
 
+def _tables_fit(q, cos, sin) -> bool:
+    """cos and sin are [T, D / 2] for q [B, T, heads, D]: row t of the tables is
+    token t's, in every sequence (the kernel sees pointers only)."""
+    return tuple(cos.shape) == tuple(sin.shape) == (q.shape[1], q.shape[3] // 2)
+
+
 def rope_cache(q, k, v, cos, sin, kc, vc, pos):
     """One launch (``bi_rope_cache``) for ``_rope`` of q and k and the writes of
     the rotated keys and the values into rows ``pos ..`` of the caches: the bits
     of those elementwise ops. Returns q rotated, ``[B, heads, T, D]``."""
     B, T, Hq, D = q.shape
     Hkv = k.shape[2]
+    if not _tables_fit(q, cos, sin):
+        raise ValueError(f"rope_cache: tables {tuple(cos.shape)} and {tuple(sin.shape)}; need ({T}, {D // 2}) each")
     out = torch.empty((B, Hq, T, D), dtype=q.dtype, device=q.device)
     strides = (_lib._c_i64 * 6)(*kc.stride()[:3], *vc.stride()[:3])
     rc = _lib.load().bi_rope_cache(q.data_ptr(), Hq * D, k.data_ptr(), Hkv * D, v.data_ptr(), Hkv * D, cos.data_ptr(),

@@ -46,3 +46,31 @@ def test_rope_cache_rejects():
     cs, c = torch.zeros(2, 32, device="cuda"), torch.zeros(1, 2, 3, 64, device="cuda")
     with pytest.raises(ValueError, match="bad shape"):
         rope_cache(q, k, k, cs, cs, c, c.clone(), 2)                         # rows past the cache
+
+
+def test_block_tables_of_another_shape_broadcast():
+    """Tables with a position per sequence ([B, 1, T, D / 2]) and with one row
+    for every token ([1, D / 2]) broadcast as in the elementwise ops: each
+    sequence gets what it gets alone with its own [T, D / 2] tables."""
+    from mlx_batch_invariant_amd import set_batch_invariant_mode
+    from mlx_batch_invariant_amd.llama import Block, LlamaConfig
+    cfg = LlamaConfig(vocab=64, hidden=256, ffn=512, layers=1, heads=4, kv_heads=2, head_dim=64, bits=None)
+    B, T, L = 3, 5, 9
+    g = gen(8)
+    blk = Block(cfg, torch.Generator(device="cuda").manual_seed(0), "cuda", torch.bfloat16)
+    x = randn((B, T, cfg.hidden), torch.bfloat16, g)
+    ang = torch.rand((B, 1, T, cfg.head_dim // 2), generator=g) * 6.3
+    ang1 = ang[0, 0, :1]
+
+    def run(x, ang):
+        cache = [torch.zeros(x.shape[0], cfg.kv_heads, L, cfg.head_dim, dtype=x.dtype, device="cuda") for _ in range(2)]
+        cos, sin = (f(ang).to(torch.bfloat16).cuda() for f in (torch.cos, torch.sin))
+        with torch.no_grad(), set_batch_invariant_mode():
+            return [blk(x, cos, sin, cache, 0), *cache]
+
+    got = run(x, ang)
+    for b in range(B):
+        for u, w in zip(got, run(x[b:b + 1], ang[b, 0])):
+            assert bits(u[b:b + 1]) == bits(w)
+    for u, w in zip(run(x, ang1), run(x, ang1.expand(T, -1))):
+        assert bits(u) == bits(w)

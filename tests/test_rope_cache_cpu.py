@@ -1,0 +1,25 @@
+"""What the fused RoPE and K/V cache write refuses, on the host: nothing is
+launched (validation comes before the library is called)."""
+
+import pytest
+import torch
+
+
+def _operands(B=2, T=3, Hq=4, Hkv=2, D=32, L=8):
+    q, k, v = (torch.zeros(B, T, h, D) for h in (Hq, Hkv, Hkv))
+    return q, k, v, torch.zeros(B, Hkv, L, D), torch.zeros(B, Hkv, L, D)
+
+
+@pytest.mark.parametrize("shape", [(2, 1, 3, 16), (1, 16), (16,), (3, 32), (4, 16), (1, 3, 16)])
+def test_tables_of_another_shape_are_refused(shape):
+    """The kernel reads [T, D / 2] from the pointers whatever the tensors are:
+    tables that broadcast (a row per sequence, one row for all tokens) or are
+    of another size never reach it."""
+    from mlx_batch_invariant_amd.llama import _tables_fit, rope_cache
+    q, k, v, kc, vc = _operands()
+    good, bad = torch.zeros(3, 16), torch.zeros(shape)
+    assert _tables_fit(q, good, good)
+    for cos, sin in ((bad, bad), (good, bad), (bad, good)):
+        assert not _tables_fit(q, cos, sin)
+        with pytest.raises(ValueError, match="tables"):
+            rope_cache(q, k, v, cos, sin, kc, vc, 0)
