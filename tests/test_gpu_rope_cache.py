@@ -1,6 +1,7 @@
 """RoPE and the K/V cache writes in one launch against the elementwise ops, bit
 for bit, over types, head sizes, token counts and cache layouts."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -38,6 +39,27 @@ def test_rope_cache_equals_elementwise(dt, B, T, Hq, Hkv, D, pos, token_major):
     assert bits(got) == bits(qw)
     for a, b in zip(base, want):
         assert bits(a) == bits(b)                                            # every other row untouched
+
+
+@pytest.mark.parametrize("pos", [3, np.int64(3), torch.tensor(3), -6])
+def test_block_position_forms(pos):
+    """Positions of any integer type, and rows counted from the cache's end."""
+    from mlx_batch_invariant_amd import set_batch_invariant_mode
+    from mlx_batch_invariant_amd.llama import Block, LlamaConfig
+    cfg = LlamaConfig(vocab=64, hidden=128, ffn=256, layers=1, heads=2, kv_heads=1, head_dim=64, bits=None)
+    g = gen(9)
+    blk = Block(cfg, torch.Generator(device="cuda").manual_seed(0), "cuda", torch.bfloat16)
+    x = randn((2, 1, cfg.hidden), torch.bfloat16, g)
+    cos, sin = randn((1, 32), torch.bfloat16, g), randn((1, 32), torch.bfloat16, g)
+    base = [randn((2, 1, 9, 64), torch.bfloat16, g) for _ in range(2)]
+
+    def run(pos):
+        cache = [c.clone() for c in base]
+        with torch.no_grad(), set_batch_invariant_mode():
+            return [blk(x, cos, sin, cache, pos), *cache]
+
+    for a, b in zip(run(pos), run(3)):                 # row -6 of 9 is row 3
+        assert bits(a) == bits(b)
 
 
 def test_rope_cache_rejects():
