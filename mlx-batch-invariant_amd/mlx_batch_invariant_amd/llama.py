@@ -18,7 +18,6 @@ element from its own inputs only.
 
 from __future__ import annotations
 
-import operator
 from dataclasses import dataclass
 
 import torch
@@ -147,8 +146,8 @@ def rope_cache(q, k, v, cos, sin, kc, vc, pos):
     out = torch.empty((B, Hq, T, D), dtype=q.dtype, device=q.device)
     strides = (_lib._c_i64 * 6)(*kc.stride()[:3], *vc.stride()[:3])
     rc = _lib.load().bi_rope_cache(q.data_ptr(), Hq * D, k.data_ptr(), Hkv * D, v.data_ptr(), Hkv * D, cos.data_ptr(),
-                                   sin.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), B, T, Hq, Hkv, D,
-                                   operator.index(pos), min(kc.shape[2], vc.shape[2]), strides, _lib.DTYPE_CODE[q.dtype], _lib.stream_of(q))
+                                   sin.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), B, T, Hq, Hkv, D, pos,
+                                   min(kc.shape[2], vc.shape[2]), strides, _lib.DTYPE_CODE[q.dtype], _lib.stream_of(q))
     _lib.check(rc, "bi_rope_cache")
     return out
 
