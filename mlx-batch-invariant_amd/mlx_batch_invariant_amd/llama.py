@@ -138,7 +138,8 @@ def _tables_fit(q, cos, sin) -> bool:
 def rope_cache(q, k, v, cos, sin, kc, vc, pos):
     """One launch (``bi_rope_cache``) for ``_rope`` of q and k and the writes of
     the rotated keys and the values into rows ``pos ..`` of the caches: the bits
-    of those elementwise ops. Returns q rotated, ``[B, heads, T, D]``."""
+    of those elementwise ops. Returns q rotated, ``[B, heads, T, D]``. The
+    caches count as changed in place (their version counters), as by the writes."""
     B, T, Hq, D = q.shape
     Hkv = k.shape[2]
     if not _tables_fit(q, cos, sin):
@@ -149,6 +150,7 @@ def rope_cache(q, k, v, cos, sin, kc, vc, pos):
                                    sin.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), B, T, Hq, Hkv, D, pos,
                                    min(kc.shape[2], vc.shape[2]), strides, _lib.DTYPE_CODE[q.dtype], _lib.stream_of(q))
     _lib.check(rc, "bi_rope_cache")
+    torch.autograd.graph.increment_version([c for c in (kc, vc) if not c.is_inference()])
     return out
 
 

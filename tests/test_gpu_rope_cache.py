@@ -62,6 +62,27 @@ def test_block_position_forms(pos):
         assert bits(a) == bits(b)
 
 
+def test_rope_cache_counts_as_an_in_place_change():
+    """The caches' version counters move, so a graph that saved a cache for its
+    backward pass notices the write; caches made in inference mode have none."""
+    from mlx_batch_invariant_amd.llama import rope_cache
+    g = gen(10)
+    q, k, v = (randn((1, 2, h, 64), torch.bfloat16, g) for h in (4, 2, 2))
+    cs = randn((2, 32), torch.bfloat16, g)
+    kc, vc = (torch.zeros(1, 2, 6, 64, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    w = torch.ones_like(kc, requires_grad=True)
+    y = (w * kc).sum()
+    before = kc._version, vc._version
+    rope_cache(q, k, v, cs, cs, kc, vc, 1)
+    assert kc._version > before[0] and vc._version > before[1]
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
+    with torch.inference_mode():
+        ki, vi = torch.zeros_like(kc), torch.zeros_like(vc)
+        rope_cache(q, k, v, cs, cs, ki, vi, 1)
+    assert bits(ki) == bits(kc) and bits(vi) == bits(vc)
+
+
 def test_rope_cache_rejects():
     from mlx_batch_invariant_amd.llama import rope_cache
     q, k = torch.zeros(1, 2, 4, 64, device="cuda"), torch.zeros(1, 2, 2, 64, device="cuda")
