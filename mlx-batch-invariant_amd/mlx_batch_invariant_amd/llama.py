@@ -123,6 +123,8 @@ def _fused_rope_ok(q, k, v, cos, sin, kc, vc, pos) -> bool:
     if any(type(t) is not torch.Tensor or not t.is_cuda or t.dtype != dt or t.device != q.device or t.data_ptr() % 16
            for t in ts):
         return False
+    if not all(_writable(c) for c in (kc, vc)):
+        return False
     # rows [b, t] at one stride with contiguous heads; contiguous tables; caches with contiguous d
     rows = all(t.is_contiguous() for t in (q, k, v, cos, sin))
     return rows and all(c.stride(3) == 1 and all(s % unit == 0 for s in c.stride()[:3])
@@ -133,6 +135,13 @@ def _tables_fit(q, cos, sin) -> bool:
     """cos and sin are [T, D / 2] for q [B, T, heads, D]: row t of the tables is
     token t's, in every sequence (the kernel sees pointers only)."""
     return tuple(cos.shape) == tuple(sin.shape) == (q.shape[1], q.shape[3] // 2)
+
+
+def _writable(c) -> bool:
+    """No stride-0 dimension (rows that share memory) and no inference tensor
+    outside inference mode: what a slice assignment into ``c`` refuses."""
+    return (all(s > 0 or n <= 1 for s, n in zip(c.stride(), c.shape))
+            and (not c.is_inference() or torch.is_inference_mode_enabled()))
 
 
 def rope_cache(q, k, v, cos, sin, kc, vc, pos):

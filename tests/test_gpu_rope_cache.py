@@ -83,6 +83,22 @@ def test_rope_cache_counts_as_an_in_place_change():
     assert bits(ki) == bits(kc) and bits(vi) == bits(vc)
 
 
+def test_block_refuses_caches_an_assignment_refuses():
+    from mlx_batch_invariant_amd import set_batch_invariant_mode
+    from mlx_batch_invariant_amd.llama import Block, LlamaConfig
+    cfg = LlamaConfig(vocab=64, hidden=128, ffn=256, layers=1, heads=2, kv_heads=1, head_dim=64, bits=None)
+    blk = Block(cfg, torch.Generator(device="cuda").manual_seed(0), "cuda", torch.bfloat16)
+    x = torch.zeros((2, 1, cfg.hidden), dtype=torch.bfloat16, device="cuda")
+    cs = torch.zeros((1, 32), dtype=torch.bfloat16, device="cuda")
+    new = lambda n: torch.zeros((n, 1, 4, 64), dtype=torch.bfloat16, device="cuda")
+    with torch.inference_mode():
+        inference = new(2)
+    for bad in (new(1).expand(2, 1, 4, 64), inference):
+        for cache in ((bad, new(2)), (new(2), bad)):
+            with torch.no_grad(), set_batch_invariant_mode(), pytest.raises(RuntimeError):
+                blk(x, cs, cs, cache, 1)
+
+
 def test_rope_cache_rejects():
     from mlx_batch_invariant_amd.llama import rope_cache
     q, k = torch.zeros(1, 2, 4, 64, device="cuda"), torch.zeros(1, 2, 2, 64, device="cuda")

@@ -23,3 +23,20 @@ def test_tables_of_another_shape_are_refused(shape):
         assert not _tables_fit(q, cos, sin)
         with pytest.raises(ValueError, match="tables"):
             rope_cache(q, k, v, cos, sin, kc, vc, 0)
+
+
+def test_caches_an_assignment_refuses():
+    """A cache broadcast over its batch, and an inference tensor outside
+    inference mode, are left to the slice assignment, which raises."""
+    from mlx_batch_invariant_amd.llama import _writable
+    c = torch.zeros(1, 2, 8, 32)
+    assert _writable(c) and _writable(c.transpose(1, 2)) and _writable(c[:, :, 2:])
+    assert _writable(c[:, :1].expand(1, 1, 8, 32))
+    assert not _writable(c.expand(3, 2, 8, 32)) and not _writable(c[:, :1].expand(1, 4, 8, 32))
+    with torch.inference_mode():
+        i = torch.zeros(1, 2, 8, 32)
+        assert _writable(i)
+    assert not _writable(i)
+    for bad in (c.expand(3, 2, 8, 32), i):
+        with pytest.raises(RuntimeError):
+            bad[:, :, 1:2] = torch.ones(bad.shape[0], 2, 1, 32)
