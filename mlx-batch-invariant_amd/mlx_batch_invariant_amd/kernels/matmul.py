@@ -90,6 +90,17 @@ def _as_row_major(b: torch.Tensor) -> torch.Tensor | None:
     return _pad_rows(b, N8)
 
 
+def _rows_within(a: torch.Tensor, K8: int) -> tuple[torch.Tensor, int]:
+    """a [Bt, M, K8] and the row stride to pass for it, below _MAX_LD: a copy when
+    the rows lie further apart. The stride of a single row is never used, and
+    torch's own notion of contiguity ignores it too."""
+    if a.shape[1] == 1:
+        return a, K8
+    if a.stride(1) >= _MAX_LD:
+        a = a.contiguous()
+    return a, a.stride(1)
+
+
 def _matmul_kn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> None:
     """out = a @ b for a [Bt, M, K] and a row-major b [Bt, K, N] (``_row_major``;
     its rows may be padded past out's N), 2-D operands taken as a batch of one."""
@@ -97,12 +108,11 @@ def _matmul_kn(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> None:
         a, b, out = a[None], b[None], out[None]
     Bt, M, K = a.shape
     N = out.shape[-1]
-    a = _prep_batched(a, (K + 7) // 8 * 8)
-    if a.stride(1) >= _MAX_LD:
-        a = a.contiguous()
+    K8 = (K + 7) // 8 * 8
+    a, lda = _rows_within(_prep_batched(a, K8), K8)
     ws_bytes = _lib.ws_bytes("bi_matmul_kn_workspace_bytes", Bt, M, N, K)
     ws = _lib.workspace(ws_bytes, a.device)
-    rc = _lib.load().bi_matmul_kn(a.data_ptr(), a.stride(0), a.stride(1), b.data_ptr(), b.stride(0), b.stride(1),
+    rc = _lib.load().bi_matmul_kn(a.data_ptr(), a.stride(0), lda, b.data_ptr(), b.stride(0), b.stride(1),
                                   out.data_ptr(), M * N, Bt, M, N, K, _lib.DTYPE_CODE[a.dtype], _lib.ptr(ws),
                                   ws_bytes, _lib.stream_of(a))
     _lib.check(rc, "bi_matmul_kn")

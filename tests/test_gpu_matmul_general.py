@@ -125,6 +125,24 @@ def test_pad_rows_copies_exactly(dt, shape, cut):
         assert bits(_pad_rows(t.expand(4, *t.shape), C)) == bits(want.expand(4, *want.shape))
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_rows_far_apart_row_major(dt):
+    """Rows 2^22 elements apart: one row in place (the last token of a prompt,
+    x[:, -1]), several rows through a copy, 2-D and batched."""
+    g = gen(11)
+    h = torch.zeros((2, 1024, 4096), dtype=DT[dt], device="cuda")
+    h[:, -1] = randn((2, 4096), DT[dt], g)
+    w = randn((4096, 72), DT[dt], g, 0.1)
+    want = _bi().batch_invariant_matmul(h[:, -1].contiguous(), w)
+    for x in (h[:1, -1], h[:, -1], h[:, -1][:, :4096]):
+        assert x.stride(0) == 1 << 22
+        assert bits(_bi().batch_invariant_matmul(x, w)) == bits(want[:x.shape[0]])
+        b3 = w.expand(1, -1, -1)
+        assert bits(_bi().batch_invariant_bmm(x[None], b3)[0]) == bits(want[:x.shape[0]])
+    b3 = w.expand(2, -1, -1).contiguous()
+    assert bits(_bi().batch_invariant_bmm(h[:, -1:], b3)) == bits(want[:, None])
+
+
 def test_odd_columns_row_major():
     """b [K, N] with an odd N or an unaligned base takes a row-padded copy."""
     g = gen(2)
