@@ -126,7 +126,8 @@ __device__ __forceinline__ void load_uniform4_i32(const int32_t* p0, const int32
 
 // K/V addressing mode of a kernel instantiation: a contiguous cache, a paged
 // one with pages of 64 keys or more, one with pages of 16 or 32 keys (every
-// aligned 16-key tile lies in one page), or one with smaller pages.
+// aligned 16-key tile lies in one page), or one with smaller pages or with rows
+// too far apart for 32-bit offsets (kFarRowBytes in bi_attn_launch.h).
 enum KvMode { kKvContig = 0, kKvPaged = 1, kKvTilePaged = 2, kKvRowPaged = 3 };
 
 // The K/V rows a kernel reads come in aligned 64-key segments (a decode wave's

@@ -83,10 +83,17 @@ __global__ void zero_counter_kernel(U* c) { *c = 0u; }
 constexpr int kDynMinRounds = 4;
 
 // K/V addressing mode (bi_attn_common.h): contiguous, pages of >= 64 keys, of
-// 16 or 32 keys, or smaller ones.
-template <class Args>
+// 16 or 32 keys, or smaller ones. The two larger page modes copy a segment's
+// (tile's) rows at 32-bit byte offsets from its first one, so pools whose keys
+// lie kFarRowBytes or more apart (position-major ones of many pages) take the
+// mode with a 64-bit address per row whatever the page size: 64 rows stay
+// below 2^30 bytes in the others.
+constexpr int64_t kFarRowBytes = (int64_t)1 << 24;
+template <typename T, class Args>
 static int kv_mode(const Args& a) {
-  return !a.table ? kKvContig : a.page_shift >= 6 ? kKvPaged : a.page_shift >= 4 ? kKvTilePaged : kKvRowPaged;
+  if (!a.table) return kKvContig;
+  if (a.page_shift < 4 || std::max(a.k_sl, a.v_sl) * (int64_t)sizeof(T) >= kFarRowBytes) return kKvRowPaged;
+  return a.page_shift >= 6 ? kKvPaged : kKvTilePaged;
 }
 
 // Paged caches always take the dynamic item order (one instantiation each).
@@ -105,7 +112,7 @@ static int launch_decode_gu(DecodeArgs& a, hipStream_t st) {
   // Enough resident workgroups to fill the chip, never more than the number
   // of possible items (every sequence at full length).
   const int64_t most = (int64_t)a.B * a.nsplit * a.Hkv * a.nchunk;
-  const int mode = kv_mode(a);
+  const int mode = kv_mode<T>(a);
   if (mode == kKvPaged) return launch_decode_paged<T, D, GU, kKvPaged>(a, most, st);
   if (mode == kKvTilePaged) return launch_decode_paged<T, D, GU, kKvTilePaged>(a, most, st);
   if (mode == kKvRowPaged) return launch_decode_paged<T, D, GU, kKvRowPaged>(a, most, st);
@@ -146,7 +153,7 @@ int launch_prefill(PrefillArgs& a, hipStream_t st) {
   const int64_t wgs = ((int64_t)a.Tq * G + 63) / 64;
   const int64_t items = wgs * a.Hkv * a.B;     // the kernel maps blocks to items per XCD
   dim3 grid((unsigned)(8 * ((items + 7) / 8)));
-  switch (kv_mode(a)) {
+  switch (kv_mode<T>(a)) {
     case kKvPaged: attn_prefill_mfma<T, D, kKvPaged><<<grid, 256, 0, st>>>(a); break;
     case kKvTilePaged: attn_prefill_mfma<T, D, kKvTilePaged><<<grid, 256, 0, st>>>(a); break;
     case kKvRowPaged: attn_prefill_mfma<T, D, kKvRowPaged><<<grid, 256, 0, st>>>(a); break;

@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma(DecodeArgs a) {
   // pages of 64 keys (kVFixed: a copy moves 64 / kCPR whole rows, so the
   // swizzle key repeats every kVPeriod copies): from this wave's first row.
   // Pages of 16 and 32 keys: from a 16-key tile's first row. The host keeps
-  // 256 rows of the V stride below 2^31 bytes.
+  // 64 rows of the V stride below 2^30 bytes.
   constexpr bool TILED = MODE == kKvTilePaged;
   constexpr bool kVFixed = (MODE == kKvContig || MODE == kKvPaged) && (64 % KV::kCPR) == 0;
   constexpr int kRowsPerCopy = kVFixed ? 64 / KV::kCPR : 1;
@@ -549,6 +549,7 @@ __global__ __launch_bounds__(256, (prefill_min_blocks<T, D, MODE, FEW>())) void 
   // the row), computed once here: no per-copy address arithmetic. Rows past
   // the sequence read as zero (their keys are masked and their weights are
   // exactly 0). The host keeps 64 rows of either stride below 2^30 bytes.
+  // Paged caches: the same from the segment's (tile's) first row.
   // When a copy moves whole rows, the swizzle key repeats every kPeriod copies:
   // the other offsets are these plus a wave-uniform row step.
   constexpr bool kFixed = 64 % KV::kCPR == 0, TILED = MODE == kKvTilePaged;

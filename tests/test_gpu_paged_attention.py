@@ -214,3 +214,43 @@ def test_prefill_few_and_many_workgroups_agree(dt, D):
     few = torch.cat([bi.batch_invariant_prefill_attention(q[i:i + 17], k[i:i + 17], v[i:i + 17], scale=D ** -0.5,
                                                           causal=True, kv_lens=lens[i:i + 17]) for i in (0, 17)])
     assert bits(many) == bits(few)
+
+
+@pytest.mark.parametrize("page_size,row_bytes", [(64, 1 << 25), (16, 1 << 27), (256, 1 << 24), (64, (1 << 24) - 256)])
+def test_pages_of_far_apart_rows(page_size, row_bytes):
+    """A position-major pool ([page_size, pages, Hkv, D]; the keys of a page
+    row_bytes apart) through the library's entry points: 64 rows span 2^30
+    bytes and more, past 32-bit offsets."""
+    bi = _bi()
+    lib, c64 = bi._lib.load(), bi._lib._c_i64
+    g = gen(page_size)
+    Hq, Hkv, L, D, dt = 8, 2, 300, 64, torch.bfloat16
+    k, v = randn((1, Hkv, L, D), dt, g), randn((1, Hkv, L, D), dt, g)
+    kp, vp, table = _paginate(k, v, page_size, g)
+    far, row = [], row_bytes // 2
+    for pool in (kp, vp):
+        P = pool.shape[0]
+        base = torch.empty(page_size * row, dtype=dt, device="cuda")
+        far.append(base.as_strided((P, Hkv, page_size, D), (Hkv * D, D, row, 1)))
+        far[-1].copy_(pool)
+    lens = torch.tensor([L], dtype=torch.int32).cuda()
+    st = [s for t in far for s in t.stride()[:3]]
+    for Tq in (1, 5):
+        q = randn((1, Hq, Tq, D), dt, g)
+        out = torch.empty_like(q)
+        common = (q.data_ptr(), far[0].data_ptr(), far[1].data_ptr(), table.data_ptr(), table.stride(0), page_size,
+                  kp.shape[0], lens.data_ptr(), out.data_ptr(), 1, Hq, Hkv)
+        Lt = table.shape[1] * page_size
+        if Tq == 1:
+            nbytes = lib.bi_attn_decode_workspace_bytes(1, Hq, Lt, D)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+            rc = lib.bi_attn_decode_paged(*common, Lt, D, (c64 * 8)(Hq * D, D, *st), D ** -0.5, bi._lib.BI_BF16,
+                                          ws.data_ptr(), nbytes, bi._lib.stream_of(q))
+        else:
+            rc = lib.bi_attn_prefill_paged(*common, Tq, Lt, D, (c64 * 9)(*q.stride()[:3], *st), 1, D ** -0.5,
+                                           bi._lib.BI_BF16, bi._lib.stream_of(q))
+        bi._lib.check(rc, "paged attention")
+        want = bi.batch_invariant_attention(q, k, v, mask="causal" if Tq > 1 else None)
+        assert bits(out) == bits(want), Tq
+    del base, far
+    torch.cuda.empty_cache()
