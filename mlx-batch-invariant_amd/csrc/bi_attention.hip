@@ -15,8 +15,8 @@
 //   combine one thread per (sequence, head, d); merges the sequence's own
 //           ceil(len/256) splits left to right and divides.
 //   prefill one 256-thread workgroup per (sequence, kv head, 64 (token, head)
-//           rows, token-major), K/V streamed through LDS in 64-key chunks,
-//           splits merged in registers.
+//           rows, token-major), K/V streamed through LDS in chunks of 64, 128
+//           or 256 keys, splits merged in registers.
 #include <mutex>
 #include <type_traits>
 
@@ -155,8 +155,8 @@ int decode_impl(const char* what, const void* q, const void* k, const void* v, c
                   (long long)strides[i]);
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(ws))
     return fail(BI_E_INVALID_ARG, "%s: q, k, v and workspace must be 16-byte aligned", what);
-  // The contiguous-cache kernel addresses a split's 256 V rows with 32-bit
-  // byte offsets.
+  // The contiguous-cache kernel addresses V rows with 32-bit byte offsets (a
+  // split's 256 rows stay below 2^31 bytes).
   if (!table && !per_key && strides[7] * (int64_t)es >= ((int64_t)1 << 23))
     return fail(BI_E_UNSUPPORTED, "%s: V position stride (%lld elements) must stay below 2^23 bytes", what,
                 (long long)strides[7]);
@@ -218,8 +218,9 @@ int prefill_impl(const char* what, const void* q, const void* k, const void* v, 
                   (long long)strides[i]);
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out))
     return fail(BI_E_INVALID_ARG, "%s: q, k, v, out must be 16-byte aligned", what);
-  // The contiguous-cache kernel addresses the 64 rows of a key chunk with
-  // 32-bit byte offsets.
+  // The contiguous-cache kernel addresses the rows of a key chunk with signed
+  // 32-bit byte offsets: up to 128 of them (the launcher takes chunks of 256
+  // keys only below 2^23 bytes).
   if (!table && !per_key && 64 * std::max(strides[5], strides[8]) * (int64_t)es >= ((int64_t)1 << 30))
     return fail(BI_E_UNSUPPORTED, "%s: K/V row strides (%lld, %lld elements) must stay below 2^24 bytes", what,
                 (long long)strides[5], (long long)strides[8]);

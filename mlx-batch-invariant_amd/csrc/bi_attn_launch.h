@@ -159,7 +159,8 @@ int launch_prefill(PrefillArgs& a, hipStream_t st) {
     case kKvRowPaged: attn_prefill_mfma<T, D, kKvRowPaged><<<grid, 256, 0, st>>>(a); break;
     default:
       if constexpr (sizeof(T) == 2 && D <= 64) {
-        if (items <= kPrefillFewItems) {
+        // (a whole split's rows at 32-bit offsets: 256 of them below 2^31 bytes)
+        if (items <= kPrefillFewItems && std::max(a.k_sl, a.v_sl) * (int64_t)sizeof(T) < ((int64_t)1 << 23)) {
           attn_prefill_mfma<T, D, kKvContig, true><<<grid, 256, 0, st>>>(a);
           break;
         }

@@ -548,7 +548,7 @@ __global__ __launch_bounds__(256, (prefill_min_blocks<T, D, MODE, FEW>())) void 
   // lane's row of the chunk times the row stride, plus its 16-byte piece of
   // the row), computed once here: no per-copy address arithmetic. Rows past
   // the sequence read as zero (their keys are masked and their weights are
-  // exactly 0). The host keeps 64 rows of either stride below 2^30 bytes.
+  // exactly 0). The host keeps a chunk's rows below 2^31 bytes at either stride.
   // Paged caches: the same from the segment's (tile's) first row.
   // When a copy moves whole rows, the swizzle key repeats every kPeriod copies:
   // the other offsets are these plus a wave-uniform row step.

@@ -406,3 +406,26 @@ def test_every_head_dim_batch_invariant(D):
     run = lambda t: _bi().batch_invariant_decode_attention(t[0], t[1], t[2], scale=D ** -0.5)
     fails = sweep((q0, k0, v0), filler, run, batches=[1, 2, 5, 16])
     assert not fails, fails
+
+
+@pytest.mark.parametrize("row_bytes", [(1 << 23) - 256, 1 << 23, (1 << 24) - 256])
+def test_prefill_rows_at_the_stride_limits(row_bytes):
+    """Contiguous caches whose keys lie as far apart as the entry point takes
+    them, on both sides of the limit of the whole-split chunks (few items,
+    head dim 64), against the compact cache."""
+    bi = _bi()
+    lib, c64 = bi._lib.load(), bi._lib._c_i64
+    q, k, v = _qkv(1, 2, 1, 5, 300, 64, "f16", seed=12)
+    far = []
+    for t in (k, v):
+        base = torch.empty(300 * row_bytes // 2, dtype=t.dtype, device="cuda")
+        far.append(base.as_strided(t.shape, (0, 0, row_bytes // 2, 1)))
+        far[-1].copy_(t)
+    out = torch.empty_like(q)
+    st = (c64 * 9)(*q.stride()[:3], *far[0].stride()[:3], *far[1].stride()[:3])
+    rc = lib.bi_attn_prefill(q.data_ptr(), far[0].data_ptr(), far[1].data_ptr(), None, out.data_ptr(), 1, 2, 1, 5, 300,
+                             64, st, 1, 0.125, bi._lib.BI_F16, bi._lib.stream_of(q))
+    bi._lib.check(rc, "bi_attn_prefill")
+    assert bits(out) == bits(bi.batch_invariant_prefill_attention(q, k, v, scale=0.125, causal=True))
+    del base, far
+    torch.cuda.empty_cache()
