@@ -34,9 +34,9 @@ SPLIT_M_MAX = 32
 
 
 def _kcontig(t: torch.Tensor) -> bool:
-    """Rows k-contiguous with 16-byte aligned row starts (what the kernel reads)."""
-    es = t.element_size()
-    return (t.stride(-1) == 1 and (t.stride(0) * es) % 16 == 0 and t.data_ptr() % 16 == 0
+    """Rows k-contiguous, 16-byte aligned, a multiple of 8 elements apart (what
+    the kernel reads)."""
+    return (t.stride(-1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
             and t.stride(0) >= t.shape[-1])
 
 
@@ -279,7 +279,7 @@ def _prep_batched(t: torch.Tensor, K8: int) -> torch.Tensor:
     batch stride (0 kept for a broadcast operand)."""
     Bt, R, K = t.shape
     es = t.element_size()
-    ok = (K8 == K and t.stride(2) == 1 and t.stride(1) >= K and (t.stride(1) * es) % 16 == 0
+    ok = (K8 == K and t.stride(2) == 1 and t.stride(1) >= K and t.stride(1) % 8 == 0
           and (t.stride(0) * es) % 16 == 0 and t.data_ptr() % 16 == 0)
     if ok:
         return t

@@ -174,10 +174,12 @@ def test_direct_call_equals_general(dt, M, N, K):
     wv.copy_(w0)
     assert bits(_matmul_direct(a, wv.t())) == bits(want)
     assert bits(_bi().batch_invariant_matmul(a, wv.t())) == bits(want)
-    if dt != "f32":
-        for y, v in [(x[1:, 1:1 + K], w0), (a0, w[1:, 4:4 + K])]:
-            assert _matmul_direct(y, v.t()) is None
-            assert bits(_bi().batch_invariant_matmul(y, v.t())) == bits(matmul_bt(y.contiguous(), v.contiguous()))
+    for y, v in [(x[1:, 1:1 + K], w0), (a0, w[1:, 4:4 + K]), (x[1:, 4:4 + K], w[1:, 4:4 + K])]:
+        assert _matmul_direct(y, v.t()) is None
+        want4 = matmul_bt(y.contiguous(), v.contiguous())
+        assert bits(_bi().batch_invariant_matmul(y, v.t())) == bits(want4)
+        y3, v3 = y.expand(2, -1, -1), v.t().expand(2, -1, -1)
+        assert bits(_bi().batch_invariant_bmm(y3, v3)) == bits(want4.expand(2, -1, -1))
     assert _matmul_direct(a0[:1].expand(2, K), w0.t()) is None
     assert _matmul_direct(a0, w0.t().double()) is None and _matmul_direct(a0.cpu(), w0.cpu().t()) is None
     assert bits(_bi().batch_invariant_matmul(a0[:1].expand(2, K), w0.t())[1]) == bits(matmul_bt(a0[:1], w0)[0])

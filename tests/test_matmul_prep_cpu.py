@@ -14,3 +14,15 @@ def test_row_stride_passed_to_the_row_major_product(M, stride):
     assert 64 <= ld < _MAX_LD and ld % 8 == 0
     assert torch.equal(y, x) and (M == 1 or y.stride(1) == ld)
     assert (y.data_ptr() == x.data_ptr()) == (M == 1 or stride < _MAX_LD)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+def test_rows_taken_in_place_are_what_the_library_takes(dt):
+    """Row strides of 4 mod 8 elements are 16-byte aligned in fp32, but the
+    library takes multiples of 8 only."""
+    from mlx_batch_invariant_amd.kernels.matmul import _kcontig, _prep_batched
+    for ld, ok in ((28, False), (32, True)):
+        x = torch.zeros((3, ld), dtype=dt)[1:, 8:16]
+        assert _kcontig(x) is ok
+        if ok:
+            assert _prep_batched(x[None], 8).data_ptr() == x.data_ptr()
