@@ -164,17 +164,23 @@ PACKED_MAX_M = 16
 _PACKED: dict = {}
 
 
-def _packed_for(bt: torch.Tensor):
-    e = _PACKED.get(bt.data_ptr())
+def _packed_at(ptr: int, N: int, K: int, ld: int, t: torch.Tensor):
+    """The copy kept for the weight [N, K] at ptr, rows ld apart, that ``t`` is a
+    view of; None if there is none or it is stale."""
+    e = _PACKED.get(ptr)
     if e is None:
         return None
     w = e[0]()
-    if w is None or w.data_ptr() != bt.data_ptr():
-        _PACKED.pop(bt.data_ptr(), None)
+    if w is None or w.data_ptr() != ptr:
+        _PACKED.pop(ptr, None)
         return None
-    if (e[1], e[2], e[3], e[4], e[5]) != (bt.shape[0], bt.shape[1], bt.stride(0), bt.dtype, bt._version):
+    if (e[1], e[2], e[3], e[4], e[5]) != (N, K, ld, t.dtype, t._version):
         return None
     return e[6]
+
+
+def _packed_for(bt: torch.Tensor):
+    return _packed_at(bt.data_ptr(), bt.shape[0], bt.shape[1], bt.stride(0), bt)
 
 
 def cache_packed_weight(weight: torch.Tensor) -> torch.Tensor:
@@ -212,18 +218,19 @@ def drop_packed_weight(weight: torch.Tensor) -> None:
 
 
 def _matmul_direct(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor | None:
-    """``bi_matmul`` for the common call: 2-D GPU operands of one dtype, ``b`` a
-    transposed view of k-contiguous rows (``W.T``), both readable in place, no
-    repacked copy to look up; None for any other call. The checks of the general
-    path on values read once, without the transposed view it builds: a call
-    whose kernel takes 4.5 us (bf16 [1, 896] @ [4864, 896].T) 11.1 -> 7.7 us."""
+    """``bi_matmul`` (``bi_matmul_packed`` for a weight with a repacked copy) for
+    the common call: 2-D GPU operands of one dtype, ``b`` a transposed view of
+    k-contiguous rows (``W.T``), both readable in place; None for any other
+    call. The checks of the general path on values read once, without the
+    transposed view it builds: a call whose kernel takes 4.5 us (bf16 [1, 896] @
+    [4864, 896].T) 11.1 -> 7.7 us."""
     if a.ndim != 2 or b.ndim != 2 or not a.is_cuda or not b.is_cuda:
         return None
     dt = a.dtype
     code = _lib.DTYPE_CODE.get(dt)
     M, K = a.shape
     Kb, N = b.shape
-    if code is None or b.dtype != dt or K != Kb or M == 0 or N == 0 or K == 0 or K % 8 or (_PACKED and M <= PACKED_MAX_M):
+    if code is None or b.dtype != dt or K != Kb or M == 0 or N == 0 or K == 0 or K % 8:
         return None
     lda, a1 = a.stride()
     b0, ldb = b.stride()
@@ -234,6 +241,12 @@ def _matmul_direct(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor | None:
     out = torch.empty((M, N), dtype=dt, device=a.device)
     ws_bytes = _lib.ws_bytes("bi_matmul_workspace_bytes", M, N, K)
     ws = _lib.workspace(ws_bytes, a.device) if ws_bytes else None
+    bp = _packed_at(pb, N, K, ldb, b) if _PACKED and M <= PACKED_MAX_M else None
+    if bp is not None:
+        rc = _lib.load().bi_matmul_packed(pa, lda, pb, ldb, bp.data_ptr(), out.data_ptr(), M, N, K, code, _lib.ptr(ws),
+                                          ws_bytes, _lib.stream_of(a))
+        _lib.check(rc, "bi_matmul_packed")
+        return out
     rc = _lib.matmul_call(pa, lda, pb, ldb, out.data_ptr(), M, N, K, code, _lib.ptr(ws), ws_bytes, _lib.stream_of(a))
     if rc:
         _lib.check(rc, "bi_matmul")

@@ -183,3 +183,31 @@ def test_direct_call_equals_general(dt, M, N, K):
     assert _matmul_direct(a0[:1].expand(2, K), w0.t()) is None
     assert _matmul_direct(a0, w0.t().double()) is None and _matmul_direct(a0.cpu(), w0.cpu().t()) is None
     assert bits(_bi().batch_invariant_matmul(a0[:1].expand(2, K), w0.t())[1]) == bits(matmul_bt(a0[:1], w0)[0])
+
+
+def test_direct_call_with_repacked_weights(monkeypatch):
+    """The direct call looks a weight's repacked copy up itself, and a copy kept
+    for one weight leaves the others' calls as they were; a stale copy is not
+    used. Same bits each way."""
+    from mlx_batch_invariant_amd import _lib
+    from mlx_batch_invariant_amd.kernels import matmul as km
+    bi = _bi()
+    g = gen(5)
+    w, other = randn((72, 512), torch.bfloat16, g), randn((72, 512), torch.bfloat16, g)
+    x = randn((17, 512), torch.bfloat16, g)
+    want, want_other = bi.batch_invariant_matmul(x, w.t()), bi.batch_invariant_matmul(x, other.t())
+    packed = []
+    real = _lib.load().bi_matmul_packed
+    monkeypatch.setattr(_lib.load(), "bi_matmul_packed", lambda *a: packed.append(a[6]) or real(*a))
+    bi.cache_packed_weight(w)
+    try:
+        for M in (1, 16, 17):
+            assert bits(km._matmul_direct(x[:M], w.t())) == bits(want[:M])
+            assert bits(km._matmul_direct(x[:M], other.t())) == bits(want_other[:M])
+        assert packed == [1, 16]
+        assert bits(km._matmul_direct(x[:4], w[:40].t())) == bits(want[:4, :40])     # another weight's shape
+        w.mul_(2)
+        assert bits(km._matmul_direct(x[:4], w.t())) == bits(bi.batch_invariant_matmul(x, w.t())[:4])
+        assert packed == [1, 16]
+    finally:
+        bi.drop_packed_weight(w)
