@@ -612,8 +612,11 @@ __global__ __launch_bounds__(256, (prefill_min_blocks<T, D, MODE, FEW>())) void 
     }
   };
   // Chunk c of the workgroup's whole sequence of chunks (the pipelined body
-  // names its next chunk itself).
-  auto issue = [&](int c) {
+  // names its next chunk itself). The lambdas of the plain body are inlined by
+  // force: with the address code of every row (pages below 16 keys) they grew
+  // past what the compiler inlines by itself at D >= 192 (fp32: D >= 96), and
+  // the workgroup's state went through scratch memory on every chunk.
+  auto issue = [&](int c) __attribute__((always_inline)) {
     if (c >= nchunks) return;
     int sp, kind, kc;
     if (c < 2 * KC * (nsplit - 1)) {
@@ -625,7 +628,7 @@ __global__ __launch_bounds__(256, (prefill_min_blocks<T, D, MODE, FEW>())) void 
     if (kind) request(std::true_type(), sp * kSplit + kc * CH, c % NBUF);
     else request(std::false_type(), sp * kSplit + kc * CH, c % NBUF);
   };
-  auto open_chunk = [&](int c) {
+  auto open_chunk = [&](int c) __attribute__((always_inline)) {
     // Chunk c landed; the min(PF - 1, nchunks - 1 - c) chunks requested after
     // it may still be in flight (copies complete in issue order).
     const int ahead = min(PF - 1, nchunks - 1 - c);
@@ -811,7 +814,7 @@ __global__ __launch_bounds__(256, (prefill_min_blocks<T, D, MODE, FEW>())) void 
     }
     }
   };
-  auto split_body_plain = [&](const int sp, auto masked) {
+  auto split_body_plain = [&](const int sp, auto masked) __attribute__((always_inline)) {
     if constexpr (!PIPE) {
     constexpr bool MASKED = decltype(masked)::value;
     const int j0 = sp * kSplit;
@@ -916,7 +919,7 @@ __global__ __launch_bounds__(256, (prefill_min_blocks<T, D, MODE, FEW>())) void 
     }
     }
   };
-  auto split_body = [&](const int sp, auto masked) {
+  auto split_body = [&](const int sp, auto masked) __attribute__((always_inline)) {
     split_body_pipe(sp, masked);
     split_body_plain(sp, masked);
   };
