@@ -124,6 +124,13 @@ __device__ __forceinline__ void load_uniform4_i32(const int32_t* p0, const int32
       : "memory");
 }
 
+// min(max(x, 0), most) of a wave-uniform x, kept in a scalar register: the
+// compiler clamps with v_med3_i32 otherwise, and a buffer resource whose size
+// is a vector register costs a readfirstlane loop around every copy.
+__device__ __forceinline__ int uniform_clamp(int x, int most) {
+  return __builtin_amdgcn_readfirstlane(min(max(x, 0), most));
+}
+
 // K/V addressing mode of a kernel instantiation: a contiguous cache, a paged
 // one with pages of 64 keys or more, one with pages of 16 or 32 keys (every
 // aligned 16-key tile lies in one page), or one with smaller pages or with rows
