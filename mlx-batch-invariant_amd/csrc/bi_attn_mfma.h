@@ -150,9 +150,9 @@ struct KVTile {
 // no workgroup that has nothing to do (with a grid over every possible split,
 // the empty workgroups of short sequences cost as much dispatch time as the
 // real work). DYN = false: workgroup w takes items w, w + P, w + 2P, ...
-// (P = grid size). DYN = true: each workgroup takes the next item from a
-// counter (a.ctr, zero at launch), so workgroups that finish early take more
-// items. Either way items come in increasing order per workgroup, which finds
+// (P = grid size). DYN = true: after item w each workgroup takes the next item
+// from a counter (a.ctr, zero at launch), so workgroups that finish early take
+// more items. Either way items come in increasing order per workgroup, which finds
 // each item's sequence by walking the lengths forward.
 // Per item: GU query heads are the 16 columns of the score tile (GU <= 16).
 // Every wave first requests all of its memory: Q^T, the K rows of its 64 keys
@@ -215,11 +215,18 @@ __global__ __launch_bounds__(256) void attn_decode_mfma(DecodeArgs a) {
   for (int64_t next = blockIdx.x;; next += gridDim.x) {
   int64_t item = next;
   if constexpr (DYN) {
-    // The end-of-item barrier below keeps thread 0 from overwriting item_s
-    // before every thread has read it.
-    if (tid == 0) item_s = atomicAdd(a.ctr, 1u);
-    __syncthreads();
-    item = item_s;
+    // The first item of workgroup w is w; the counter hands out the items from
+    // gridDim.x on. (It serves some 55 requests a us, one by one, which bounds
+    // a decode of many short rows, and the more so the more workgroups are
+    // resident when each takes its first item from it too. fp16 D = 32, B = 16,
+    // 4,096 keys, pages of 16 / 256: 58 / 55 us so, now 39.) The end-of-item
+    // barrier below keeps thread 0 from overwriting item_s before every thread
+    // has read it.
+    if (next >= gridDim.x) {
+      if (tid == 0) item_s = atomicAdd(a.ctr, 1u);
+      __syncthreads();
+      item = (int64_t)gridDim.x + item_s;
+    }
   }
   // Advance to the sequence holding `item` (uniform per workgroup). A length
   // outside [0, L] is clamped, so no key past the cache is ever read.

@@ -272,3 +272,24 @@ def test_small_pages_equal_contiguous_at_every_head_dim(dt, D):
         mask = "causal" if Tq > 1 else None
         got = bi.batch_invariant_paged_attention(q, kp, vp, table, lens, mask=mask)
         assert bits(got) == bits(bi.batch_invariant_attention(q, k, v, kv_lens=lens, mask=mask))
+
+
+@pytest.mark.parametrize("B,L", [(3, 40), (5, 1500), (150, 3000)])
+def test_paged_decode_item_order(B, L):
+    """Fewer work items than workgroups, about as many, and several times as
+    many (first items by workgroup, the rest from the counter), with empty and
+    ragged sequences, against each sequence alone."""
+    bi = _bi()
+    g = gen(B)
+    Hq, Hkv, D = 8, 4, 64
+    k, v = randn((B, Hkv, L, D), torch.bfloat16, g), randn((B, Hkv, L, D), torch.bfloat16, g)
+    q = randn((B, Hq, 1, D), torch.bfloat16, g)
+    lens = torch.randint(0, L + 1, (B,), generator=g).to(torch.int32)
+    lens[0], lens[B // 2], lens[-1] = 0, L, 1
+    kp, vp, table = _paginate(k, v, 32, g)
+    got = bi.batch_invariant_paged_attention(q, kp, vp, table, lens.cuda())
+    for b in {0, 1, B // 2, B // 3, B - 1}:
+        n = int(lens[b])
+        want = (bi.batch_invariant_attention(q[b:b + 1], k[b:b + 1, :, :n], v[b:b + 1, :, :n]) if n
+                else torch.zeros_like(q[:1]))
+        assert bits(got[b:b + 1]) == bits(want), (b, n)
