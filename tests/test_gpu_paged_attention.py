@@ -258,14 +258,16 @@ def test_pages_of_far_apart_rows(page_size, row_bytes):
 
 @pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
 @pytest.mark.parametrize("D", [32, 64, 96, 128, 192, 256])
-def test_small_pages_equal_contiguous_at_every_head_dim(dt, D):
-    """Pages below 16 keys (a row address per key): several splits, a
-    partial last chunk, ragged lengths, decode and prefill."""
+@pytest.mark.parametrize("page_size", [8, 32, 128])
+def test_pages_equal_contiguous_at_every_head_dim(dt, D, page_size):
+    """Every addressing form (a row address per key, 16-key tiles, 64-key
+    segments): several splits, a partial last chunk, ragged lengths, decode and
+    prefill."""
     bi = _bi()
     g = gen(D)
     B, Hq, Hkv, L = 2, 4, 2, 617
     k, v = randn((B, Hkv, L, D), DT[dt], g), randn((B, Hkv, L, D), DT[dt], g)
-    kp, vp, table = _paginate(k, v, 8, g)
+    kp, vp, table = _paginate(k, v, page_size, g)
     lens = torch.tensor([617, 300], dtype=torch.int32).cuda()
     for Tq in (1, 40):
         q = randn((B, Hq, Tq, D), DT[dt], g)
