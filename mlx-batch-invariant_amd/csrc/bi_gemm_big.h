@@ -106,9 +106,11 @@ constexpr int big_threads() { return 64 * BigTile<WM, BN>::kWaves; }
 //   kBColumns b[k][n] (row-major right-hand side, n contiguous), a batch.
 enum BMode { kBPlain = 0, kBRows = 1, kBColumns = 2 };
 
-// Element strides between the slices of a batch (kBRows, kBColumns).
+// Element strides between the slices of a batch (kBRows, kBColumns), and the K
+// chunks per slice of a launch that splits K (gemm_tall).
 struct BatchStride {
   int64_t a, b, out;
+  int chunks = 1;
 };
 
 // kBColumns stage: 64 k rows of BN columns, 2 BN bytes each, 16-byte chunk c of

@@ -14,8 +14,21 @@ constexpr int kGenCols[kGenForms] = {64, 64, 64, 128, 128};
 
 struct GenPlan {
   int form = kGen64x64;
-  int chunks = 1, cg = 0;   // K chunks of cg groups (tall forms, one matrix)
+  int chunks = 1, cg = 0;   // K chunks of cg groups (tall forms, row-major B)
 };
+
+// fold_groups over a batch: slice blockIdx.y of part[slice][g][M N].
+template <typename T>
+__global__ __launch_bounds__(256) void fold_groups_batch(const float* __restrict__ part, T* __restrict__ out,
+                                                         int64_t MN, int G, int64_t out_stride) {
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= MN) return;
+  part += blockIdx.y * MN * G;
+  float total = 0.0f;
+#pragma unroll 8
+  for (int g = 0; g < G; ++g) total = total + part[(int64_t)g * MN + idx];
+  out[blockIdx.y * out_stride + idx] = to_store<T>(total);
+}
 
 static inline int64_t gen_tiles(int64_t batch, int64_t M, int64_t N, int form) {
   return batch * ceil_div(M, kGenRows[form]) * ceil_div(N, kGenCols[form]);
@@ -34,9 +47,13 @@ static inline int64_t gen_tiles(int64_t batch, int64_t M, int64_t N, int form) {
 //   [333, 896, K 4864]       51 / 26 / 38 / 53   (42 tiles of 128 x 64; 64 x 64 in 7 K chunks 23)
 // 256 x 128 runs one workgroup per CU, so it wants several rounds of tiles or a
 // long K; 128 x 64 runs two and hides each other's prologue and stores. Rows up
-// to 64 take the tall tiles (64 x [64, 128, K 512]: 64x64 8.7, 128x64 19). One
-// row-major B with few tiles also splits K: [64, 4096, K 4096] 42 -> 17 us in 8
-// chunks, [1, 1024, K 4096] 31 -> 6.2 in 16, [16, 14336, K 4096] 31 -> 28 in 2.
+// to 64 take the tall tiles (64 x [64, 128, K 512]: 64x64 8.7, 128x64 19), more
+// rows only with K split. A row-major B with few tiles splits K: [64, 4096, K
+// 4096] 42 -> 17 us in 8 chunks, [1, 1024, K 4096] 31 -> 6.2 in 16, [16, 14336,
+// K 4096] 31 -> 28 in 2; and so does a small batch, whose chain of K stages is
+// otherwise longer than one launch per matrix with K split was: 2 x [1, 64, K
+// 65536] 75 by matrix, 462 unsplit, 18 split; 2 x [64, 64, K 4096] 26 / 44 / 9.7;
+// 4 x [512, 128, K 16384] 145 / 167 / 57; 2 x [33, 64, K 1000] 38 / 14 / 9.5.
 static inline GenPlan gen_plan(int64_t batch, int64_t M, int64_t N, int64_t K, BMode mode) {
   GenPlan p;
   const int G = ceil_div(K, kGroupK);
@@ -49,9 +66,9 @@ static inline GenPlan gen_plan(int64_t batch, int64_t M, int64_t N, int64_t K, B
   else if (t64 > 256 && t128 <= 256 && K >= 1024) p.form = kGen128x128;
   else if (t64 >= 48) p.form = kGen128x64;
   else p.form = kGen64x64;
-  if (p.form <= kGen64x64 && batch == 1 && mode == kBColumns) {
-    const int64_t t = gen_tiles(1, M, N, p.form);
-    if (t < 256 && G >= 2) {
+  if (p.form <= kGen64x64 && mode == kBColumns) {
+    const int64_t t = gen_tiles(batch, M, N, p.form);
+    if (batch == 1 ? t < 256 && G >= 2 : t <= (M <= 16 ? 31 : 64) && G >= 4) {
       p.cg = ceil_div(G, std::min<int64_t>(G, ceil_div(512, t)));
       p.chunks = ceil_div(G, p.cg);
     }
@@ -94,15 +111,20 @@ template <typename T, BMode MODE, int TI, int RMAX>
 static void launch_gen_tall(const T* a, int64_t lda, const T* b, int64_t ldb, T* out, float* ws, int batch,
                             BatchStride bs, int M, int N, int K, const GenPlan& p, hipStream_t st) {
   const int G = ceil_div(K, kGroupK);
-  if (p.chunks > 1) {
-    const dim3 grid(ceil_div(N, 64), ceil_div(M, 16 * TI), p.chunks);
-    gemm_tall<T, TI, 1, 4, 64, true, RMAX, MODE><<<grid, 256, 0, st>>>(a, lda, b, ldb, out, ws, M, N, K, G, p.cg, bs);
-    const int64_t MN = (int64_t)M * N;
-    fold_groups<T><<<(unsigned)((MN + 255) / 256), 256, 0, st>>>(ws, out, MN, G);
-  } else {
-    const dim3 grid(ceil_div(N, 64), ceil_div(M, 16 * TI), batch);
-    gemm_tall<T, TI, 1, 4, 64, false, RMAX, MODE><<<grid, 256, 0, st>>>(a, lda, b, ldb, out, ws, M, N, K, G, G, bs);
+  if constexpr (MODE == kBColumns) {
+    if (p.chunks > 1) {                       // few tiles: batch * chunks stays below 65,536
+      const dim3 grid(ceil_div(N, 64), ceil_div(M, 16 * TI), batch * p.chunks);
+      bs.chunks = p.chunks;
+      gemm_tall<T, TI, 1, 4, 64, true, RMAX, MODE><<<grid, 256, 0, st>>>(a, lda, b, ldb, out, ws, M, N, K, G, p.cg, bs);
+      const int64_t MN = (int64_t)M * N;
+      const dim3 fold((unsigned)((MN + 255) / 256), batch);
+      if (batch == 1) fold_groups<T><<<fold, 256, 0, st>>>(ws, out, MN, G);
+      else fold_groups_batch<T><<<fold, 256, 0, st>>>(ws, out, MN, G, bs.out);
+      return;
+    }
   }
+  const dim3 grid(ceil_div(N, 64), ceil_div(M, 16 * TI), batch);
+  gemm_tall<T, TI, 1, 4, 64, false, RMAX, MODE><<<grid, 256, 0, st>>>(a, lda, b, ldb, out, ws, M, N, K, G, G, bs);
 }
 
 template <typename T, BMode MODE>

@@ -64,8 +64,8 @@ struct TallCfg {
   static __device__ __forceinline__ int slot(int r, int c) { return c ^ (r & (kChunks - 1)); }
 };
 
-// BMODE (bi_gemm_big.h) other than kBPlain: a batch of matrices (unsplit:
-// grid.z is the batch; SPLIT: one matrix), any K % 8 == 0, B as bt[n][k] or
+// BMODE (bi_gemm_big.h) other than kBPlain: a batch of matrices (grid.z is the
+// batch; SPLIT: the batch times the K chunks, part[slice][g][m][n]), any K % 8 == 0, B as bt[n][k] or
 // b[k][n]. 64-k stages and 64 columns, so a stage's B is 64 rows of 128 bytes
 // in either layout.
 template <typename T, int TI, int WM, int WN, int SK, bool SPLIT, int RMAX = 12, int BMODE = kBPlain>
@@ -75,10 +75,20 @@ __global__ __launch_bounds__(256) void gemm_tall(const T* __restrict__ a, int64_
   static_assert(sizeof(T) == 2, "gemm_tall: 2-byte element types only");
   constexpr bool GEN = BMODE != kBPlain, KN = BMODE == kBColumns;
   static_assert(!GEN || (SK == 64 && WN == 4), "gemm_tall: 64 x 64 B stages outside kBPlain");
+  int zc = blockIdx.z;                                              // SPLIT: K chunk
   if constexpr (GEN && !SPLIT) {
     a += blockIdx.z * bs.a;
     bt += blockIdx.z * bs.b;
     out += blockIdx.z * bs.out;
+  }
+  if constexpr (GEN && SPLIT) {
+    if ((int)gridDim.z > bs.chunks) {                               // (no division for one matrix)
+      const int64_t slice = zc / bs.chunks;
+      zc %= bs.chunks;
+      a += slice * bs.a;
+      bt += slice * bs.b;
+      part += slice * G * M * N;
+    }
   }
   typedef TallCfg<TI, WM, WN, SK, RMAX> C;
   constexpr int SPG = C::kStagesPerGroup;
@@ -91,7 +101,7 @@ __global__ __launch_bounds__(256) void gemm_tall(const T* __restrict__ a, int64_
   const int r = lane % 16, q = lane / 16;
   const int wm = wave / WN, wn = wave % WN;
   const int n0 = blockIdx.x * C::kBN, m0 = blockIdx.y * C::kBM;
-  const int g_begin = SPLIT ? blockIdx.z * CG : 0;
+  const int g_begin = SPLIT ? zc * CG : 0;
   const int g_end = SPLIT ? min(G, g_begin + CG) : G;
   const int st0 = SPG * g_begin, nst = SPG * (g_end - g_begin);  // stages of this workgroup
   const int st_valid = (K + SK - 1) / SK;                           // stages with k inside K (global index)

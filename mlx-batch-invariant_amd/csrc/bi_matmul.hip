@@ -227,9 +227,9 @@ extern "C" int bi_matmul_batched(const void* a, int64_t a_batch_stride, int64_t 
 // The right-hand side stored row-major, b[k][n]: the same tiles with the B
 // stages copied as k rows and transposed by the LDS reads.
 extern "C" size_t bi_matmul_kn_workspace_bytes(int64_t batch, int64_t M, int64_t N, int64_t K) {
-  if (batch != 1 || M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
-  const bi::GenPlan p = bi::gen_plan(1, M, N, K, bi::kBColumns);
-  return p.chunks > 1 ? (size_t)((K + bi::kGroupK - 1) / bi::kGroupK * M * N) * sizeof(float) : 0;
+  if (batch < 1 || M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
+  const bi::GenPlan p = bi::gen_plan(batch, M, N, K, bi::kBColumns);
+  return p.chunks > 1 ? (size_t)(batch * ((K + bi::kGroupK - 1) / bi::kGroupK) * M * N) * sizeof(float) : 0;
 }
 
 extern "C" int bi_matmul_kn(const void* a, int64_t a_batch_stride, int64_t lda, const void* b, int64_t b_batch_stride,

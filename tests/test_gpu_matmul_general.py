@@ -211,3 +211,21 @@ def test_direct_call_with_repacked_weights(monkeypatch):
         assert packed == [1, 16]
     finally:
         bi.drop_packed_weight(w)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("B,M,N,K", [(2, 1, 64, 1032), (31, 16, 64, 1024), (32, 16, 64, 1024), (3, 33, 130, 4100),
+                                     (64, 64, 8, 776), (65, 64, 64, 776), (2, 65, 130, 20000), (4, 200, 72, 1280),
+                                     (17, 129, 64, 1000), (2, 300, 96, 520)])
+def test_small_batches_with_long_k(dt, B, M, N, K):
+    """Row-major batches that split K and their neighbours that do not: the
+    lines of the rule, partial groups, several K chunks per slice, a broadcast
+    operand."""
+    g = gen(B + M + K)
+    a = randn((B, M, K), DT[dt], g)
+    b = randn((B, K, N), DT[dt], g, 0.1)
+    got = _bi().batch_invariant_bmm(a, b)
+    one = _bi().batch_invariant_bmm(a, b[:1].expand(B, K, N))
+    for i in {0, B // 2, B - 1}:
+        _check_rows(got[i], a[i], b[i].t(), [0, M // 2, M - 1])
+        _check_rows(one[i], a[i], b[0].t(), [M - 1])
