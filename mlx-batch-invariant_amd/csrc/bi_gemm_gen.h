@@ -44,7 +44,7 @@ static inline int64_t gen_tiles(int64_t batch, int64_t M, int64_t N, int form) {
 //   [515, 4096, K 4096]      81 / 38 / 34 / 46   (96)
 //   [2000, 4096, K 4096]     194 / 82 / 84 / 64  (256)
 //   [3000, 14336, K 4096]    920 / 470 / 442 / 376
-//   [333, 896, K 4864]       51 / 26 / 38 / 53   (42 tiles of 128 x 64; 64 x 64 in 7 K chunks 23)
+//   [333, 896, K 4864]       51 / 26 / 38 / 53   (42 tiles of 128 x 64; 64 x 64 in 7 K chunks 23, row-major B only)
 // 256 x 128 runs one workgroup per CU, so it wants several rounds of tiles or a
 // long K; 128 x 64 runs two and hides each other's prologue and stores. Rows up
 // to 64 take the tall tiles (64 x [64, 128, K 512]: 64x64 8.7, 128x64 19), more
@@ -73,6 +73,7 @@ static inline GenPlan gen_plan(int64_t batch, int64_t M, int64_t N, int64_t K, B
       p.chunks = ceil_div(G, p.cg);
     }
   }
+  if (M > 64 && p.form == kGen64x64 && p.chunks == 1) p.form = kGen128x64;
   return p;
 }
 
