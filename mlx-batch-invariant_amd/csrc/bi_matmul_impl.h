@@ -1258,9 +1258,17 @@ static inline bool mid_may_split(int64_t M, int64_t N, int64_t K) {
 //   [4096, 14336] M = 255  57.5 / 79.4 / 79.3 / 117  -> 47.2 / 57.2 / 49.3 / 69.9
 //   [1024, 4096]  M = 255  18.2 / 20.8 / 18.5 / 23.0 -> 9.3 / 12.0 / 10.6 / 17.1
 // K split stays for [1024, 4096] M = 64 (8.4 against 9.3), [4096, 14336] M =
-// 32 (22.5 against 27.4). Interleaving the dequantization with the MFMAs by
-// hand, or the other scheduler and register forms, measured no faster.
-static inline MidPlan mid_plan(int64_t M, int64_t N, int64_t K) {
+// 32 (22.5 against 27.4). With 20 - 32 groups it stays too where whole K is the
+// longer chain (split / whole): 33 - 64 rows of 8-bit codes in the MLX layout
+// (mlx8, the slowest to load; one 64-row block reads them once): [4096, 8192]
+// M = 33 / 64 22.4 / 29.4 and 26.8 / 30.3, [2048, 6144] M = 64 18.3 / 22.8 (not
+// where two row tiles fill the chip: [8192, 8192] M = 64 47.5 / 33.8); and
+// at exactly 128 workgroups, above 24 groups, for mlx8 ([1024, 8192] M = 128
+// 22.4 / 28.7; 4-bit 20.7 / 20.6; [1000, 4608] 19.5 / 18.3) and up to 64 rows
+// ([2048, 8192] M = 64 4-bit 18.0 / 20.6, 8-bit g128 packed 16.2 / 18.6; [4096,
+// 8192] M = 32 4-bit 19.3 / 20.7). Interleaving the dequantization with the
+// MFMAs by hand, or the other scheduler and register forms, measured no faster.
+static inline MidPlan mid_plan(int64_t M, int64_t N, int64_t K, bool mlx8) {
   MidPlan p;
   if (M <= 4 || M >= kBigMinM || N <= 0 || K <= 0 || K % kGroupK) return p;
   const int G = (int)(K / kGroupK);
@@ -1272,7 +1280,9 @@ static inline MidPlan mid_plan(int64_t M, int64_t N, int64_t K) {
     int mt = 1;
     while (mt <= 4 && cb * ceil_div(M, 16 * mt) > kMidOneRound) mt *= 2;
     const int64_t wg = mt <= 4 ? cb * ceil_div(M, 16 * mt) : 0;
-    const bool whole = G <= 32 ? wg >= 128 : !mid_may_split(M, N, K);
+    const bool whole = G > 32 || (mlx8 && mt == 1 && G >= 20 && M > 32 && M <= 64)
+                           ? !mid_may_split(M, N, K)
+                           : wg >= (G > 24 && (mlx8 || M <= 64) ? 129 : 128);
     if (mt <= 4 && G >= 2 && whole) {
       p.form = kMidInterleaved;
       p.mt = mt;
@@ -1411,7 +1421,7 @@ static int run_gemm(const T* a, int64_t lda, const BSrc& bsrc, T* out, int M, in
     }
   }
   if constexpr (BSrc::kMeta) {
-    const MidPlan mp = mid_plan(M, N, K);
+    const MidPlan mp = mid_plan(M, N, K, BSrc::kBits == 8);
     if (use_mid<T, BSrc>(mp, lda, a)) {
       launch_mid<T, BSrc>(a, lda, bsrc, out, ws, M, N, K, G, mp, st);
       return bi_host::launch_status(what);
@@ -1561,7 +1571,7 @@ int run_quant_packed_gs(const void* x, int64_t ldx, const uint32_t* w, const voi
     // 14336] M = 32 / 64 30.4-31.1 / 43.1 -> 24.1-24.3 / 36.1 us, [4096,
     // 4096] M = 32 / 64 15.8-16.1 / 17.8 -> 14.0-14.2 / 16.7 us (same box,
     // bits equal): their per-CU load rate, not the arithmetic, bounds them.
-    MidPlan mp = mid_plan(M, N, K);
+    MidPlan mp = mid_plan(M, N, K, false);
     // 33-64 rows that the plan splits over K (a long K) run unsplit on the
     // copy as 32-row blocks when that gives at least 128 workgroups: [4096,
     // 14336] M = 64 32.4 -> 29.9 us (8-bit g128 35.8 -> 31.5; the same group

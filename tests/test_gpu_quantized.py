@@ -552,3 +552,22 @@ def test_quantized_mid_m_row_tiles(bits_, gs, packed, N, K):
         for r in [q for q in alone if q < M]:
             assert bits(got[r:r + 1]) == alone[r], (M, r)
     bi.drop_packed(wq)
+
+
+@pytest.mark.parametrize("bits_,packed", [(4, False), (8, False), (8, True)])
+@pytest.mark.parametrize("N,K", [(1000, 4096), (1000, 4608)])
+def test_quantized_mid_m_at_128_workgroups(bits_, packed, N, K):
+    """16 column blocks around M = 128: K whole or split by how its codes are
+    laid out and by 16 or 18 K groups, against the rows computed alone."""
+    bi = _bi()
+    wq, s, b = (t.cuda() for t in _qweights(N, K, bits_, 64, "f16", seed=bits_ + K))
+    x = randn((129, K), torch.float16, gen(N + K))
+    run = lambda xx: bi.batch_invariant_quantized_matmul(xx, wq, s, b, group_size=64, bits=bits_)
+    alone = {r: bits(run(x[r:r + 1])) for r in (0, 111, 127, 128)}
+    if packed:
+        bi.cache_packed(wq, s, b, group_size=64, bits=bits_)
+    for M in (112, 113, 128, 129):
+        got = run(x[:M])
+        for r in [q for q in alone if q < M]:
+            assert bits(got[r:r + 1]) == alone[r], (M, r)
+    bi.drop_packed(wq)
