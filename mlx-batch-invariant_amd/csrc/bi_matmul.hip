@@ -16,7 +16,7 @@ size_t split_ws_bytes(int64_t M, int64_t N, int64_t K, bool dense) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const bool small_split = bi::use_split(M, (int)G) && !bi::use_wg(M, (int)G);
   const bool tall_split = dense && bi::tall_plan(M, N, K).chunks > 1;
-  const bool mid_split = dense ? bi::few_columns_plan(M, N, K).use : bi::mid_plan(M, N, K, true).chunks > 1;
+  const bool mid_split = dense ? bi::few_columns_plan(M, N, K).use : bi::mid_may_split(M, N, K);
   if (!small_split && !tall_split && !mid_split) return 0;
   return (size_t)(G * M * N) * sizeof(float);
 }

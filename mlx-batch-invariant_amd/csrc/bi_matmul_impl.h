@@ -1227,9 +1227,8 @@ static inline MidPlan few_columns_plan(int64_t M, int64_t N, int64_t K) {
   return p;
 }
 
-// Few (64-column, row block) tiles: what a plan that keeps K whole has to beat.
-// (mid_plan decides, and the workspace query reports the group partials of its
-// mlx8 plan, which splits every shape that another layout's does.)
+// Whether a call may split K: the shapes for which the workspace query reports
+// the group partials (a fixed part of the C ABI; mid_plan splits fewer).
 static inline bool mid_may_split(int64_t M, int64_t N, int64_t K) {
   if (M <= 4 || M >= kBigMinM || N <= 0 || K <= 0 || K % kGroupK || K / kGroupK < 2) return false;
   const int64_t cb = ceil_div(N, 64);

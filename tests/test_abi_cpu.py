@@ -352,14 +352,3 @@ def test_row_major_rhs_checks():
     assert not _row_major(torch.zeros(64, 60, dtype=torch.bfloat16)) and not _row_major(h[:, ::2])
     assert not _row_major(h[:1].expand(64, 64)) and not _row_major(torch.zeros(3 * 68, dtype=torch.float16)
                                                                    .as_strided((3, 8, 8), (68, 8, 1)))
-
-
-def test_quantized_workspace_follows_the_plan():
-    """Group partials are reported where a launch of some layout splits K:
-    shapes that run whole in all of them need none."""
-    lib = _lib.load()
-    need = lib.bi_quantized_matmul_workspace_bytes
-    for M, N, K in ((64, 4096, 4096), (32, 4096, 4096), (255, 1024, 4096), (128, 1024, 4096), (160, 2048, 8192)):
-        assert need(M, N, K) == 0, (M, N, K)
-    for M, N, K in ((64, 4096, 8192), (128, 1024, 8192), (64, 2048, 8192), (64, 1024, 4096), (32, 4096, 14336)):
-        assert need(M, N, K) == K // 256 * M * N * 4, (M, N, K)
