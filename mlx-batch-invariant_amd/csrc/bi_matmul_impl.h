@@ -1227,8 +1227,11 @@ static inline MidPlan few_columns_plan(int64_t M, int64_t N, int64_t K) {
   return p;
 }
 
-// Whether a call may split K: the shapes for which the workspace query reports
-// the group partials (a fixed part of the C ABI; mid_plan splits fewer).
+// The shapes for which the workspace query reports the group partials: every
+// shape that some plan splits, and more, which run whole and leave their
+// workspace unused ([4096, 4096] M = 64: 16 MB). The answer for a shape is what
+// callers have sized and saved workspaces by, and a test holds it, so it is not
+// narrowed as plans change.
 static inline bool mid_may_split(int64_t M, int64_t N, int64_t K) {
   if (M <= 4 || M >= kBigMinM || N <= 0 || K <= 0 || K % kGroupK || K / kGroupK < 2) return false;
   const int64_t cb = ceil_div(N, 64);
