@@ -342,7 +342,7 @@ def test_row_major_rhs_checks():
     assert call(ldb=1 << 26) == -2 and call(lda=1 << 22) == -2
     assert lib.bi_matmul_kn_workspace_bytes(1, 1, 1024, 4096) == 16 * 1024 * 4     # 16 chunks of one group
     assert call(M=1, N=1024, K=4096, lda=4096, ldb=1024, obs=1024) == -3
-    assert lib.bi_matmul_kn_workspace_bytes(2, 1, 1024, 4096) == 0                 # a batch never splits K
+    assert lib.bi_matmul_kn_workspace_bytes(2, 1, 1024, 4096) == 0                 # 32 tiles of up to 16 rows: not split
     assert lib.bi_matmul_kn_workspace_bytes(1, 512, 4096, 4096) == 0
     h = torch.zeros(64, 64, dtype=torch.bfloat16)
     b3 = torch.zeros(3, 64, 64, dtype=torch.float16)
