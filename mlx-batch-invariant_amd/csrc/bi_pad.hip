@@ -8,13 +8,16 @@
 // an element at a time). One thread per 16 output bytes, the source read as
 // 16 bytes at its own alignment (global loads need none); the last chunk of a
 // row by element. bf16 [14299, 4067]: zero fill and copy 60 us, this 38.
+#include <algorithm>
+
 #include "bi_common.h"
 
 namespace bi {
 
 template <typename E>
 __global__ __launch_bounds__(256) void pad_rows_kernel(const E* __restrict__ in, int64_t bs, int64_t rs,
-                                                       E* __restrict__ out, int64_t rows, int cols, int chunks) {
+                                                       E* __restrict__ out, int64_t rows, int64_t out_bs, int cols,
+                                                       int chunks) {
   constexpr int kE = 16 / (int)sizeof(E);
   const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (id >= rows * chunks) return;
@@ -30,7 +33,7 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const E* __restrict__ in,
     for (int i = 0; i < kE; ++i) e[i] = c + i < cols ? src[i] : (E)0;
     __builtin_memcpy(&v, e, 16);
   }
-  *reinterpret_cast<u32x4*>(out + ((int64_t)blockIdx.y * rows + row) * chunks * kE + c) = v;
+  *reinterpret_cast<u32x4*>(out + blockIdx.y * out_bs + row * chunks * kE + c) = v;
 }
 
 }  // namespace bi
@@ -47,22 +50,27 @@ extern "C" int bi_pad_rows(const void* in, int64_t batch_stride, int64_t row_str
   if (batch == 0 || rows == 0 || cols_out == 0) return BI_OK;
   if (!in || !out || !aligned16(out) || reinterpret_cast<uintptr_t>(in) % (unsigned)elem_bytes)
     return fail(BI_E_INVALID_ARG, "%s: null or misaligned operand", what);
-  const int64_t chunks = cols_out / unit, blocks = (rows * chunks + 255) / 256;
-  if (cols_out > 0x7fffffffLL || rows > 0x7fffffffLL || blocks > 0x7fffffffLL)
-    return fail(BI_E_UNSUPPORTED, "%s: shape too large", what);
+  const int64_t chunks = cols_out / unit;
+  if (cols_out > 0x7fffffffLL || rows > 0x7fffffffLL) return fail(BI_E_UNSUPPORTED, "%s: shape too large", what);
+  // A launch holds fewer than 2^32 threads (64 GiB of output): larger operands
+  // take several.
+  const int64_t most = std::max<int64_t>(1, ((int64_t)1 << 31) / chunks);
   hipStream_t st = static_cast<hipStream_t>(stream);
   for (int64_t b = 0; b < batch; b += 65535) {
-    const dim3 grid((unsigned)blocks, (unsigned)(batch - b < 65535 ? batch - b : 65535));
-    const char* src = static_cast<const char*>(in) + b * batch_stride * elem_bytes;
-    char* dst = static_cast<char*>(out) + b * rows * cols_out * elem_bytes;
-    if (elem_bytes == 2)
-      bi::pad_rows_kernel<uint16_t><<<grid, 256, 0, st>>>(reinterpret_cast<const uint16_t*>(src), batch_stride,
-                                                          row_stride, reinterpret_cast<uint16_t*>(dst), rows, (int)cols,
-                                                          (int)chunks);
-    else
-      bi::pad_rows_kernel<uint32_t><<<grid, 256, 0, st>>>(reinterpret_cast<const uint32_t*>(src), batch_stride,
-                                                          row_stride, reinterpret_cast<uint32_t*>(dst), rows, (int)cols,
-                                                          (int)chunks);
+    for (int64_t r = 0; r < rows; r += most) {
+      const int64_t n = std::min(most, rows - r);
+      const dim3 grid((unsigned)((n * chunks + 255) / 256), (unsigned)std::min<int64_t>(batch - b, 65535));
+      const char* src = static_cast<const char*>(in) + (b * batch_stride + r * row_stride) * elem_bytes;
+      char* dst = static_cast<char*>(out) + (b * rows + r) * cols_out * elem_bytes;
+      if (elem_bytes == 2)
+        bi::pad_rows_kernel<uint16_t><<<grid, 256, 0, st>>>(reinterpret_cast<const uint16_t*>(src), batch_stride,
+                                                            row_stride, reinterpret_cast<uint16_t*>(dst), n,
+                                                            rows * cols_out, (int)cols, (int)chunks);
+      else
+        bi::pad_rows_kernel<uint32_t><<<grid, 256, 0, st>>>(reinterpret_cast<const uint32_t*>(src), batch_stride,
+                                                            row_stride, reinterpret_cast<uint32_t*>(dst), n,
+                                                            rows * cols_out, (int)cols, (int)chunks);
+    }
   }
   return launch_status(what);
 }

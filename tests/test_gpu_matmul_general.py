@@ -229,3 +229,22 @@ def test_small_batches_with_long_k(dt, B, M, N, K):
     for i in {0, B // 2, B - 1}:
         _check_rows(got[i], a[i], b[i].t(), [0, M // 2, M - 1])
         _check_rows(one[i], a[i], b[0].t(), [M - 1])
+
+
+def test_pad_rows_past_one_launch():
+    """More 16-byte pieces than one launch has threads (2^32): 64 GiB of output
+    from one broadcast row, the rows at both ends of every launch."""
+    from mlx_batch_invariant_amd.kernels.matmul import _pad_rows
+    free = torch.cuda.mem_get_info()[0]
+    if free < 90 << 30:
+        pytest.skip(f"{free >> 30} GiB of GPU memory free, 90 needed")
+    R, step = (1 << 32) // 3 + 1000, (1 << 31) // 3
+    row = torch.arange(1, 18, dtype=torch.bfloat16, device="cuda")
+    out = _pad_rows(row.expand(R, 17), 24)
+    want = torch.zeros(24, dtype=torch.bfloat16, device="cuda")
+    want[:17] = row
+    for r in (0, 1, step - 1, step, 2 * step - 1, 2 * step, R - 1):
+        assert bits(out[r]) == bits(want), r
+    assert bool((out[::4099] == want).all())
+    del out
+    torch.cuda.empty_cache()
