@@ -76,7 +76,7 @@ extern "C" int bi_rope_cache(const void* q, int64_t q_row, const void* k, int64_
   if (dtype != BI_BF16 && dtype != BI_F16 && dtype != BI_F32)
     return fail(BI_E_UNSUPPORTED, "%s: unknown dtype %d", what, dtype);
   if (B > 0x7fffffffLL || T > 0x7fffffffLL || max_len > 0x7fffffffLL || Hq > 65536 || Hkv > 65536 || D > 65536 ||
-      B * T > ((int64_t)1 << 31) || B * T * (Hq + 2 * Hkv) * (D / 16) > ((int64_t)1 << 39))
+      B * T > ((int64_t)1 << 31) || B * T * (Hq + 2 * Hkv) * (D / 16) > ((int64_t)1 << 32) - 256)  // threads
     return fail(BI_E_UNSUPPORTED, "%s: shape too large", what);
   if (B == 0 || T == 0) return BI_OK;
   const int64_t unit = 16 / (int64_t)dtype_size(dtype);

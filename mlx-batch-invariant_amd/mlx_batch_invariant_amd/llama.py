@@ -125,6 +125,8 @@ def _fused_rope_ok(q, k, v, cos, sin, kc, vc, pos) -> bool:
         return False
     if not all(_writable(c) for c in (kc, vc)):
         return False
+    if q.numel() + 2 * k.numel() > 16 * ((1 << 32) - 256):               # elements of one launch
+        return False
     # rows [b, t] at one stride with contiguous heads; contiguous tables; caches with contiguous d
     rows = all(t.is_contiguous() for t in (q, k, v, cos, sin))
     return rows and all(c.stride(3) == 1 and all(s % unit == 0 for s in c.stride()[:3])

@@ -285,6 +285,16 @@ def test_dense_pack_sizes_and_rejections():
     assert lib.bi_matmul_packed(p, 12, p, 12, None, p, 2, 4, 12, 2, None, 0, None) == -1
 
 
+def test_rope_cache_launch_limit():
+    """More chunks than one launch has threads (2^32) are refused, not run in part."""
+    lib = _lib.load()
+    p = ctypes.c_void_p(16)
+    st = (ctypes.c_int64 * 6)(*([128] * 6))
+    call = lambda B, T: lib.bi_rope_cache(p, 128, p, 128, p, 128, p, p, p, p, p, B, T, 1, 1, 128, 0, 1 << 22, st, 2, None)
+    assert call(0, 1 << 20) == 0
+    assert call(2048, 1 << 18) == -2 and "too large" in _err(lib)        # 2048 x 2^18 x 3 heads x 8 chunks
+
+
 def test_split_size_routing():
     """split_size other than 256 runs the per-key kernels (the only ones that
     take it); asking the matrix-core kernels for it is an error."""
