@@ -137,7 +137,8 @@ int bi_matmul_batched(const void* a, int64_t a_batch_stride, int64_t lda, const 
  * 16-byte aligned operands, (K + 512) * ldb < 2^30; when K is not a multiple of
  * 8 the elements [K, 8 ceil(K / 8)) of every a row must be zero. The bits are
  * bi_matmul's on the transposed operand. Workspace: fp32 group partials when
- * a small product or batch splits K (bi_matmul_kn_workspace_bytes).
+ * a small product or batch splits K (bi_matmul_kn_workspace_bytes); a batch
+ * without it runs unsplit, a single product needs it.
  * Replaces: the transposed copy a row-major right-hand side needed before
  * bi_matmul; the reference reads either layout through strides
  * (kernels/matmul.py:279-340). */

@@ -54,7 +54,7 @@ static inline int64_t gen_tiles(int64_t batch, int64_t M, int64_t N, int form) {
 // otherwise longer than one launch per matrix with K split was: 2 x [1, 64, K
 // 65536] 75 by matrix, 462 unsplit, 18 split; 2 x [64, 64, K 4096] 26 / 44 / 9.7;
 // 4 x [512, 128, K 16384] 145 / 167 / 57; 2 x [33, 64, K 1000] 38 / 14 / 9.5.
-static inline GenPlan gen_plan(int64_t batch, int64_t M, int64_t N, int64_t K, BMode mode) {
+static inline GenPlan gen_plan(int64_t batch, int64_t M, int64_t N, int64_t K, BMode mode, bool split = true) {
   GenPlan p;
   const int G = ceil_div(K, kGroupK);
   p.cg = G;
@@ -66,7 +66,7 @@ static inline GenPlan gen_plan(int64_t batch, int64_t M, int64_t N, int64_t K, B
   else if (t64 > 256 && t128 <= 256 && K >= 1024) p.form = kGen128x128;
   else if (t64 >= 48) p.form = kGen128x64;
   else p.form = kGen64x64;
-  if (p.form <= kGen64x64 && mode == kBColumns) {
+  if (split && p.form <= kGen64x64 && mode == kBColumns) {
     const int64_t t = gen_tiles(batch, M, N, p.form);
     if (batch == 1 ? t < 256 && G >= 2 : t <= (M <= 16 ? 31 : 64) && G >= 4) {
       p.cg = ceil_div(G, std::min<int64_t>(G, ceil_div(512, t)));

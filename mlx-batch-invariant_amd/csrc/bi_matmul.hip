@@ -258,11 +258,13 @@ extern "C" int bi_matmul_kn(const void* a, int64_t a_batch_stride, int64_t lda, 
                 "%s: b of K=%lld rows of %lld elements (K + 512 rows must stay below 2^30 elements, lda below 2^22)", what,
                 (long long)K, (long long)ldb);
   const size_t need = bi_matmul_kn_workspace_bytes(batch, M, N, K);
-  if (need && (!ws || ws_bytes < need || !aligned16(ws)))
+  const bool no_ws = need && (!ws || ws_bytes < need || !aligned16(ws));
+  if (no_ws && batch == 1)
     return fail(BI_E_WORKSPACE, "%s: 16-byte aligned workspace of %zu bytes required, got %zu", what, need,
                 ws ? ws_bytes : (size_t)0);
+  // (A batch without its workspace runs with K whole, as before batches split.)
   const auto run = dtype == BI_BF16 ? bi::gen_matmul_bf16 : bi::gen_matmul_f16;
-  return run(bi::kBColumns, a, lda, b, ldb, out, ws, batch,
+  return run(bi::kBColumns, a, lda, b, ldb, out, no_ws ? nullptr : ws, batch,
              bi::BatchStride{a_batch_stride, b_batch_stride, out_batch_stride}, (int)M, (int)N, (int)K,
              static_cast<hipStream_t>(stream), what);
 }

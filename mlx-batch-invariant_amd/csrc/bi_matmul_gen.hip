@@ -8,7 +8,7 @@ namespace bi {
 template <typename T>
 static int gen_matmul(BMode mode, const void* a, int64_t lda, const void* b, int64_t ldb, void* out, void* ws,
                       int64_t batch, BatchStride bs, int M, int N, int K, hipStream_t st, const char* what) {
-  const GenPlan p = gen_plan(batch, M, N, K, mode);
+  const GenPlan p = gen_plan(batch, M, N, K, mode, ws != nullptr);
   const T* ap = static_cast<const T*>(a);
   const T* bp = static_cast<const T*>(b);
   T* op = static_cast<T*>(out);

@@ -231,6 +231,26 @@ def test_small_batches_with_long_k(dt, B, M, N, K):
         _check_rows(one[i], a[i], b[0].t(), [M - 1])
 
 
+@pytest.mark.parametrize("M", [1, 40, 200])
+def test_small_batch_without_workspace(M):
+    """A batch that splits K runs unsplit, with the same bits, where the caller
+    brings no workspace, a short one or a misaligned one."""
+    bi = _bi()
+    lib = bi._lib.load()
+    g = gen(M)
+    B, N, K = 2, 72, 2048
+    a, b = randn((B, M, K), torch.bfloat16, g), randn((B, K, N), torch.bfloat16, g, 0.1)
+    want = bi.batch_invariant_bmm(a, b)
+    need = lib.bi_matmul_kn_workspace_bytes(B, M, N, K)
+    assert need > 0
+    ws = torch.empty(need + 16, dtype=torch.uint8, device="cuda")
+    for ptr, n in ((None, 0), (ws.data_ptr(), need - 16), (ws.data_ptr() + 8, need), (ws.data_ptr(), need)):
+        out = torch.empty_like(want)
+        bi._lib.check(lib.bi_matmul_kn(a.data_ptr(), M * K, K, b.data_ptr(), K * N, N, out.data_ptr(), M * N, B, M, N, K,
+                                       bi._lib.BI_BF16, ptr, n, bi._lib.stream_of(a)), "bi_matmul_kn")
+        assert bits(out) == bits(want)
+
+
 def test_pad_rows_past_one_launch():
     """More 16-byte pieces than one launch has threads (2^32): 64 GiB of output
     from one broadcast row, the rows at both ends of every launch."""
