@@ -1246,9 +1246,10 @@ static inline bool mid_may_split(int64_t M, int64_t N, int64_t K) {
 //   * the fewest row tiles per workgroup (1, 2, 4) that keep the grid within
 //     one workgroup per CU run the K-interleaved eight-wave kernel, unless
 //     that leaves fewer than 128 workgroups (more than 32 groups:
-//     mid_may_split), when K is split;
+//     mid_may_split; 20 - 32 groups: below), when K is split;
 //   * larger grids run four waves per workgroup, MT = 2 .. 5 row tiles by the
-//     fitted cost 5 + 1.85 MT us per row block (one K = 4096 pass at cb = 224).
+//     fitted cost 5 + 1.85 MT us per row block (one K = 4096 pass at cb = 224);
+//     more than five row tiles are not built.
 // Both with two A stages and two groups of codes in flight: 16 MT (32 MT) KB
 // of LDS, so two to five workgroups share a CU where a deeper ring held one or
 // two and left a second round. Measured, old plan -> this one, us, 4-bit g64
